@@ -117,6 +117,32 @@ def test_quantizer_strided_rows(pkg, dev):
     assert torch.equal(q, qr) and torch.equal(s, sr)
 
 
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("dim", [1, 2, 3, 8, 50, 100, 127, 128, 257, 260, 512, 516, 520, 1024, 1032, 2048, 2056])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_quantizer_chunk_edges(pkg, dev, dt, dim, shift):
+    """Widths at the edges of each load width and of the chunks per lane, base pointers off by one
+    element, row counts that leave a wavefront part empty, and quotients on and beside rounding
+    boundaries (the bytes are those of the division, bit for bit)."""
+    print(f"quantize dt={dt} dim={dim} shift={shift}", flush=True)
+    rng = np.random.default_rng(dim + shift)
+    for rows in (1, 261):
+        x = rng.standard_normal((rows, dim)).astype(np.float32)
+        x[::3] = rng.integers(-127, 127, x[::3].shape) + 0.5 * rng.integers(0, 2, x[::3].shape)
+        x[::3, 0] = 127.0
+        x[1::6] = np.nextafter(np.rint(x[1::6] * 30) + np.float32(0.5), rng.choice([-1e9, 1e9], x[1::6].shape).astype(np.float32))
+        x[1::6, 0] = 127.0
+        x[2::7] *= np.float32(1e-9)  # scales at their lower limit
+        base = torch.zeros(rows * dim + shift, dtype=TORCH_DT[dt], device=dev)
+        w = base[shift:].view(rows, dim)
+        w.copy_(torch.from_numpy(x))
+        q, s = pkg.quantize_embedding_int8(w)
+        qr, sr = reference_quantize(w)
+        torch.cuda.synchronize()
+        assert torch.equal(s.view(torch.int32), sr.view(torch.int32))
+        assert torch.equal(q, qr)
+
+
 # ------------------------------------------------------------------------------------------------
 # pooling
 # ------------------------------------------------------------------------------------------------
