@@ -16,7 +16,7 @@ void clear_error();
 int check_launch(const char* what);
 
 // Bags per tile of a launch whose rows are `emb_dim` elements of `table_dtype` (aligned
-// buffers), or 0 when such rows take the element-wise kernel, which follows no tile order.
+// buffers), or 0 when such rows take the ragged kernel, which follows no tile order.
 int order_bags_per_tile(int32_t table_dtype, int32_t emb_dim);
 
 // Dispatch-order buffer layout shared by the device pass and the host builder:

@@ -60,13 +60,14 @@
 //     `count`; the long kernel reads `total`. A call therefore leaves `count` at zero for the next.
 //   * Tiles are renumbered so each of the 8 XCDs (own L2 each) works on a contiguous range of
 //     tiles, i.e. on a few fields at a time.
-//   * Rows that are not whole lane vectors, or misaligned buffers, use an element-wise kernel
-//     (one wavefront per bag, element order, never split).
+//   * Rows of any other width, or misaligned buffers, take the ragged kernel: chunks of one lane
+//     vector at any alignment, the last one ending with the row (element order, never split).
 // All kernels write disjoint output rows and combine partial sums in a fixed order, so results
 // are deterministic run to run.
 #include <stdint.h>
 #include <string.h>
 
+#include <algorithm>
 #include <type_traits>
 #include <vector>
 
@@ -88,6 +89,9 @@ constexpr int kBinThreads = 256;
 constexpr int64_t kLongBlocksMax = 1024;  // workgroups of the long kernel (they loop over the list)
 constexpr int kMaxFields = 64;
 constexpr int64_t kNoLimit = INT64_MAX;
+// Longest bag pooled by one subgroup of a ranked tile (longer ones are split over the wavefront), and
+// longest whose mean div_by_count takes.
+constexpr int64_t kMaxShortBag = int64_t{1} << 24;
 
 // One lane's row vector (Elem<TT>::kVecBytes bytes; an 8-byte vector fills .x and .y).
 template <typename TT>
@@ -122,8 +126,8 @@ struct FieldDesc {
   int32_t out_col;     // first output column
   int32_t gidx;        // field index used for offsets / val_base
   uint32_t span_bytes; // bytes from row 0 to the end of the last row, when below 4 GiB (else 0)
-  int32_t lanes_log2;  // mixed-width launches: the field's rows are 1 << lanes_log2 lanes x one vector
-  int32_t tile_begin;  // mixed-width launches: the field's first tile (fields in tile order)
+  int32_t lanes;       // mixed-width launches: log2 of the field's lanes (one vector each); ragged: its chunks
+  int32_t tile_begin;  // mixed-width and ragged launches: the field's first tile (fields in tile order)
 };
 
 struct PoolParams {
@@ -974,7 +978,7 @@ __global__ void __launch_bounds__(kMainThreads) pool_kernel(const PoolParams p) 
 }
 
 // Main kernel of a mixed-width launch: the fields' rows differ in width but each is one lane
-// vector per lane (LANES = 1 << lanes_log2). Fields own consecutive ranges of tiles; a workgroup
+// vector per lane (LANES = 1 << lanes). Fields own consecutive ranges of tiles; a workgroup
 // finds its tile's field (one compare per lane and a ballot) and runs that width's tile code, so
 // fields of every width share one launch (and one binning pass and one list kernel).
 template <typename TT, typename OT, bool BUF>
@@ -992,7 +996,7 @@ __global__ void __launch_bounds__(kMainThreads) pool_mixed_kernel(const PoolPara
   const int first = lane < p.num_fields ? p.f[lane].tile_begin : INT32_MAX;
   const int fi = __popcll(__ballot(first <= tile)) - 1;  // field 0 starts at tile 0
   const int local = tile - p.f[fi].tile_begin;
-  switch (p.f[fi].lanes_log2) {
+  switch (p.f[fi].lanes) {
     case 2: pool_tile<TT, OT, 4, 1, BUF>(p, fi, local, s.l2); break;
     case 3: pool_tile<TT, OT, 8, 1, BUF>(p, fi, local, s.l3); break;
     case 4: pool_tile<TT, OT, 16, 1, BUF>(p, fi, local, s.l4); break;
@@ -1408,15 +1412,15 @@ __device__ __forceinline__ void store_bag_rt(const PoolParams& p, int64_t b, int
   store_out<VEC>(reinterpret_cast<OT*>(p.out) + b * p.out_row_stride + out_col + sl * VEC, r, p.stream_out);
 }
 
-// ... or, in a mixed launch, each field's own (one lane vector per lane, 1 << lanes_log2 lanes
-// per row, kMixedLo <= lanes_log2 <= kMixedHi), chosen at run time.
+// ... or, in a mixed launch, each field's own (one lane vector per lane, 1 << lanes lanes
+// per row, kMixedLo <= lanes <= kMixedHi), chosen at run time.
 template <typename TT, typename OT, int LW>
 struct MixedRows {
   static constexpr int VEC = Elem<TT>::kVecBytes / Elem<TT>::kBytes;
   static constexpr int DMAX = Shape<TT, 1 << kMixedHi, 1>::D;
   __device__ static __forceinline__ void split(const PoolParams& p, int fi, int64_t b, int64_t bs, int64_t be,
                                                int wave, float* s_red, unsigned int* ids) {
-    const int ll = p.f[fi].lanes_log2;
+    const int ll = p.f[fi].lanes;
     const int D = VEC << ll;
     const int sl = lane_id() & ((1 << ll) - 1);
     const bool g0 = lane_id() < (1 << ll);
@@ -1447,7 +1451,7 @@ struct MixedRows {
   }
   __device__ static __forceinline__ void one(const PoolParams& p, int fi, int64_t b, int64_t bs, int64_t be,
                                              unsigned int* ids) {
-    const int ll = p.f[fi].lanes_log2;
+    const int ll = p.f[fi].lanes;
     float pa[VEC];
 #pragma unroll
     for (int i = 0; i < VEC; ++i) pa[i] = 0.f;
@@ -1516,71 +1520,265 @@ __global__ void __launch_bounds__(LW * kWave) pool_long_kernel(const PoolParams 
   }
 }
 
-// Element-wise kernel for any row width / alignment: one wavefront per bag, rows accumulated in
-// order, 4 columns per lane per pass (int8 rows: fma with the row's scale).
-template <typename TT, typename OT>
-__global__ void __launch_bounds__(kMainThreads) pool_generic_kernel(const PoolParams p) {
-  constexpr int NC = 4;
-  const int tile = block_tile();
-  const int fi = field_of_tile(p, tile);
+// ---------------------------------------------------------------------------------------------
+// Ragged rows: any width and alignment. A row of `dim` elements is read as n = ceil(dim / C) chunks
+// of one lane vector (C elements), the last one moved back to end with the row, so that every load
+// stays inside the row and needs no tail; the elements that two chunks share are added and stored
+// twice, alike. n lanes hold a row (n need not be a power of two) and R = 64 / n consecutive bags (at
+// most 32) are pooled side by side, each in element order and never split. Rows narrower
+// than a vector are read element by element (C = 1); rows of more than 64 chunks are walked 64 chunks
+// at a time. Chunks need only their element's alignment (16-byte loads and stores at any address of
+// global memory, through under-aligned types).
+// Bound by latency (offsets, ids and rows are dependent loads) and by vector-ALU issue: the next
+// stage's ids are loaded under this stage's rows and 4 rows per lane are in flight; one round of
+// bags per tile, as narrow rows' tiles are the launch's longest chains (two length-ranked rounds
+// took 30 us). 28 fields of 10 to 300 bf16 columns, 2,047 samples, mean length 8: 26 us; one
+// wavefront per bag with 2-byte loads and one row in flight took 117. kRaggedRows 8: the same time.
+// ---------------------------------------------------------------------------------------------
+constexpr int kRaggedRows = 4;   // rows in flight per lane
+constexpr int kRaggedIds = 256;  // row ids staged at once: a power of two of them per bag, at most 64
+
+// Elements per chunk, chunks per row and bags per tile of rows of `dim` elements.
+template <typename TT>
+__host__ __device__ constexpr int ragged_vec() { return Elem<TT>::kVecBytes / Elem<TT>::kBytes; }
+__host__ __device__ inline int ragged_chunks(int dim, int vec) { return dim < vec ? dim : (dim + vec - 1) / vec; }
+// Bags side by side: a tile is one round of them (narrow rows' tiles are the launch's longest chains).
+__host__ __device__ inline int ragged_side(int chunks) { return chunks < 2 ? 32 : (chunks < kWave ? kWave / chunks : 1); }
+
+struct RaggedLds {
+  unsigned int ids[kRaggedIds];
+  int64_t len[32];
+  int64_t start[32];
+};
+
+// Vectors at any element's alignment.
+typedef u32x4 u32x4_any __attribute__((aligned(1)));
+typedef u32x2 u32x2_any __attribute__((aligned(1)));
+
+// C elements at an address aligned to one of them.
+template <typename TT, int C>
+__device__ __forceinline__ uint4 load_ragged(const char* p) {
+  constexpr int EB = Elem<TT>::kBytes;
+  if constexpr (C == 1) {
+    if constexpr (EB == 4) return make_uint4(*reinterpret_cast<const uint32_t*>(p), 0u, 0u, 0u);
+    else if constexpr (EB == 2) return make_uint4(*reinterpret_cast<const uint16_t*>(p), 0u, 0u, 0u);
+    else return make_uint4(*reinterpret_cast<const uint8_t*>(p), 0u, 0u, 0u);
+  } else if constexpr (C * EB == 16) {
+    const u32x4 v = *reinterpret_cast<const u32x4_any*>(p);
+    return make_uint4(v.x, v.y, v.z, v.w);
+  } else {
+    const u32x2 v = *reinterpret_cast<const u32x2_any*>(p);
+    return make_uint4(v.x, v.y, 0u, 0u);
+  }
+}
+
+template <typename TT, int C>
+__device__ __forceinline__ void acc_ragged(float* a, const uint4& v, float s) {
+  if constexpr (C > 1) {
+    acc_row<TT>(a, v, s);
+  } else if constexpr (Quantized<TT>::value) {
+    a[0] = __builtin_fmaf(static_cast<float>(static_cast<int8_t>(v.x)), s, a[0]);
+  } else {
+    a[0] += Elem<TT>::load(&v.x);
+  }
+}
+
+// C results at an address aligned to one of them; STREAM: non-temporal.
+template <int C, bool STREAM, typename OT>
+__device__ __forceinline__ void store_ragged(OT* dst, const float* r) {
+  const auto put16 = [&](int e, u32x4 v) {
+    u32x4_any* const q = reinterpret_cast<u32x4_any*>(dst + e);
+    if constexpr (STREAM) __builtin_nontemporal_store(v, q);
+    else *q = v;
+  };
+  if constexpr (C == 1) {
+    store_one(dst, r[0], STREAM);
+  } else if constexpr (sizeof(OT) == 4) {
+#pragma unroll
+    for (int i = 0; i < C; i += 4)
+      put16(i, u32x4{__float_as_uint(r[i]), __float_as_uint(r[i + 1]), __float_as_uint(r[i + 2]), __float_as_uint(r[i + 3])});
+  } else {
+    uint32_t w[C / 2];
+#pragma unroll
+    for (int i = 0; i < C / 2; ++i) {
+      if constexpr (__is_same(OT, bf16_t)) w[i] = pack_bf16x2(r[2 * i], r[2 * i + 1]);
+      else w[i] = pack_f16x2(r[2 * i], r[2 * i + 1]);
+    }
+    if constexpr (C == 8) {
+      put16(0, u32x4{w[0], w[1], w[2], w[3]});
+    } else {
+      static_assert(C == 4, "a chunk is one lane vector");
+      u32x2_any* const q = reinterpret_cast<u32x2_any*>(dst);
+      if constexpr (STREAM) __builtin_nontemporal_store(u32x2{w[0], w[1]}, q);
+      else *q = u32x2{w[0], w[1]};
+    }
+  }
+}
+
+// BUF: rows at 4-byte aligned addresses of a float table of less than 4 GiB: byte offsets are staged
+// in place of row ids and the rows read with buffer loads, past a bag's end at the table's end, which
+// reads zeros without a memory request.
+template <typename TT, typename OT, int C, bool BUF>
+__device__ __forceinline__ void ragged_tile(const PoolParams& p, int fi, int local_tile, RaggedLds& s) {
+  constexpr int U = kRaggedRows;
+  static_assert(8 % U == 0, "U divides the ids staged per bag (8 or more: at most 32 bags side by side)");
+  constexpr int kIdsPerLane = kRaggedIds / kWave;
+  static_assert(!BUF || C * Elem<TT>::kBytes == 16, "buffer loads are 16-byte chunks");
+  const unsigned int span = p.f[fi].span_bytes;
+  const Rsrc rsrc = make_rsrc(p.f[fi].table, BUF ? span : 0u);
   const char* const table = p.f[fi].table;
+  const float* const row_scale = p.f[fi].row_scale;
   const int64_t max_row = p.f[fi].max_row;
   const int64_t row_bytes = p.f[fi].row_bytes;
   const int dim = p.f[fi].dim;
-  const int out_col = p.f[fi].out_col;
+  const int chunks = p.f[fi].lanes;
+  const int n = chunks < kWave ? chunks : kWave;
+  const int R = ragged_side(chunks);
+  const int lq_max = 31 - __builtin_clz(static_cast<unsigned>(kRaggedIds / R));
+  const int lq = lq_max < 6 ? lq_max : 6;  // ids staged per bag: 1 << lq (R << lq <= kRaggedIds)
   const int lane = lane_id();
-  const int64_t b = static_cast<int64_t>(tile - fi * p.tiles_per_field);
-  if (b >= p.batch) return;
-  int64_t start, end;
-  bag_range(p, p.f[fi].gidx, b, start, end);
+  const int g = lane / n, sl = lane - g * n;
+  const int64_t b0 = static_cast<int64_t>(local_tile) * R;
+
+  // lane i describes bag b0 + i
+  const int nv = p.batch - b0 < R ? static_cast<int>(p.batch - b0) : R;
+  int64_t start = 0, end = 0;
+  if (lane < nv) bag_range(p, p.f[fi].gidx, b0 + lane, start, end);
   const int64_t L = end - start;
-  OT* o = reinterpret_cast<OT*>(p.out) + b * p.out_row_stride + out_col;
-  for (int c0 = 0; c0 < dim; c0 += kWave * NC) {
-    float acc[NC];
+  if (lane < nv) {
+    s.len[lane] = L;
+    s.start[lane] = start;
+  }
+  __syncthreads();  // one wavefront per workgroup
+
+  // Stages: rows c0 .. c0 + (1 << lq) - 1 of every bag, column block cb; at least one per block. The
+  // next stage's ids are loaded before this stage's rows, so they arrive under them.
+  int64_t id[kIdsPerLane];
+  unsigned int staged = 0;  // bit i: id[i] is a row of a bag
+  auto load_ids = [&](int64_t c0) {
+    staged = 0;
 #pragma unroll
-    for (int i = 0; i < NC; ++i) acc[i] = 0.f;
-    for (int64_t c = start; c < end; c += kWave) {
-      int64_t roff = 0;
-      float rsc = 0.f;
-      if (c + lane < end) {
-        const int64_t row = clamp_i64(load_index(p, c + lane), 0, max_row);
-        roff = row * row_bytes;
-        if constexpr (Quantized<TT>::value) rsc = p.f[fi].row_scale[row];
+    for (int i = 0; i < kIdsPerLane; ++i) {
+      const int e = lane + i * kWave;
+      const int b = e >> lq;
+      const int64_t at = c0 + (e & ((1 << lq) - 1));
+      if (b < nv && at < s.len[b]) {
+        id[i] = load_index(p, s.start[b] + at);
+        staged |= 1u << i;
       }
-      const int n = static_cast<int>(end - c < kWave ? end - c : kWave);
-      for (int k = 0; k < n; ++k) {
-        const int64_t ro = shfl_i64(roff, k);
-        const float sk = Quantized<TT>::value ? __int_as_float(shfl_i32(__float_as_int(rsc), k)) : 1.f;
+    }
+  };
+  const bool has = g < nv;
+  const int gi = has ? g : 0;  // lanes without a bag follow bag 0's ids and store nothing
+  const int64_t Lb = has ? s.len[gi] : 0;
+  int cb = 0, col = 0;
+  int64_t c0 = 0;
+  unsigned int col_bytes = 0;
+  float acc[C];
+  load_ids(0);
+  while (cb < chunks) {
+    if (c0 == 0) {
+      col = (cb + sl) * C;  // first element of this lane's chunk
+      if (col > dim - C) col = dim - C;
+      col_bytes = static_cast<unsigned int>(col * Elem<TT>::kBytes);
 #pragma unroll
-        for (int i = 0; i < NC; ++i) {
-          const int col = c0 + i * kWave + lane;
-          if (col < dim) {
-            const float x = Elem<TT>::load(table + ro + static_cast<int64_t>(col) * Elem<TT>::kBytes);
-            if constexpr (Quantized<TT>::value) acc[i] = __builtin_fmaf(x, sk, acc[i]);
-            else acc[i] += x;
-          }
+      for (int i = 0; i < C; ++i) acc[i] = 0.f;
+    }
+    __syncthreads();  // the last stage's reads are done
+#pragma unroll
+    for (int i = 0; i < kIdsPerLane; ++i) {
+      const int e = lane + i * kWave;
+      if (e < (R << lq)) {
+        // past a bag: the table's end, or row 0, whose data is not used
+        const unsigned int r = static_cast<unsigned int>(clamp_i64(id[i], 0, max_row));
+        s.ids[e] = staged >> i & 1u ? (BUF ? r * static_cast<unsigned int>(row_bytes) : r) : (BUF ? span : 0u);
+      }
+    }
+    __syncthreads();
+    int64_t c0n = c0 + (int64_t{1} << lq);
+    int cbn = cb;
+    if (__ballot(c0n < L) == 0) {  // no bag has more rows
+      c0n = 0;
+      cbn = cb + kWave;
+    }
+    if (cbn < chunks) load_ids(c0n);
+    const int64_t left = Lb - c0;
+    const int live = left < 0 ? 0 : (left < (int64_t{1} << lq) ? static_cast<int>(left) : 1 << lq);
+    for (int k = 0; __ballot(k < live) != 0; k += U) {
+      uint4 v[U];
+      float sc[U];
+      unsigned int r[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) r[u] = s.ids[(gi << lq) + k + u];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if constexpr (BUF) {
+          v[u] = buffer_load16(rsrc, r[u] + col_bytes);
+        } else {
+          v[u] = load_ragged<TT, C>(table + static_cast<uint64_t>(r[u]) * static_cast<uint64_t>(row_bytes) + col_bytes);
+        }
+        sc[u] = 1.f;
+        if constexpr (Quantized<TT>::value) sc[u] = row_scale[r[u]];
+      }
+      __builtin_amdgcn_sched_barrier(0);  // issue every load of the step before consuming any
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if constexpr (!BUF) {
+          const bool act = k + u < live;
+          v[u].x = act ? v[u].x : 0u;
+          v[u].y = act ? v[u].y : 0u;
+          v[u].z = act ? v[u].z : 0u;
+          v[u].w = act ? v[u].w : 0u;
+          if constexpr (Quantized<TT>::value) sc[u] = act ? sc[u] : 0.f;
+        }
+        acc_ragged<TT, C>(acc, v[u], sc[u]);
+      }
+    }
+    if (c0n == 0) {  // the bags' last stage
+      if (p.pooling == CTI_EBAG_MEAN && Lb > 0) {
+        if (Lb <= kMaxShortBag) {
+          div_by_count<C>(acc, 1.0 / static_cast<double>(Lb), static_cast<float>(Lb));
+        } else {
+#pragma unroll
+          for (int i = 0; i < C; ++i) acc[i] = acc[i] / static_cast<float>(Lb);
         }
       }
-    }
-#pragma unroll
-    for (int i = 0; i < NC; ++i) {
-      const int col = c0 + i * kWave + lane;
-      if (col < dim) {
-        float r = acc[i];
-        if (p.pooling == CTI_EBAG_MEAN && L > 0) r = r / static_cast<float>(L);
-        round_like_reference<TT, 1>(p, &r);
-        store_one(o + col, r, p.stream_out);
+      round_like_reference<TT, C>(p, acc);
+      if (has && cb + sl < chunks) {
+        OT* const dst = reinterpret_cast<OT*>(p.out) + (b0 + g) * p.out_row_stride + p.f[fi].out_col + col;
+        with_stream(p.stream_out, [&](auto stream) { store_ragged<C, decltype(stream)::value>(dst, acc); });
       }
     }
+    c0 = c0n;
+    cb = cbn;
   }
+}
+
+template <typename TT, typename OT>
+__global__ void __launch_bounds__(kMainThreads) pool_ragged_kernel(const PoolParams p) {
+  __shared__ RaggedLds s;
+  // Workgroup i runs on XCD i % 8, which takes the i % 8-th eighth of every field's tiles, field after
+  // field (tile_begin counts positions of that list): the XCDs get like shares of every row width, and
+  // the narrowest rows start first (the host's order), whose many bags per tile are the longest chains.
+  const int pos = static_cast<int>(blockIdx.x) >> 3, x = static_cast<int>(blockIdx.x) & 7;
+  const int lane = lane_id();
+  const int first = lane < p.num_fields ? p.f[lane].tile_begin : INT32_MAX;
+  const int fi = __popcll(__ballot(first <= pos)) - 1;  // field 0 starts at position 0
+  const int next = fi + 1 < p.num_fields ? p.f[fi + 1].tile_begin : p.num_tiles >> 3;
+  const int local = x * (next - p.f[fi].tile_begin) + pos - p.f[fi].tile_begin;
+  if (static_cast<int64_t>(local) * ragged_side(p.f[fi].lanes) >= p.batch) return;  // up to 7 per field
+  if constexpr (!Quantized<TT>::value) {
+    if (p.f[fi].span_bytes) return ragged_tile<TT, OT, ragged_vec<TT>(), true>(p, fi, local, s);
+  }
+  if (p.f[fi].dim >= ragged_vec<TT>()) ragged_tile<TT, OT, ragged_vec<TT>(), false>(p, fi, local, s);
+  else ragged_tile<TT, OT, 1, false>(p, fi, local, s);
 }
 
 // ---------------------------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------------------------
 int lanes_of(int variant) { return variant <= 6 ? (1 << variant) : 64; }
-int bags_per_tile(int variant) {
-  if (variant == kVarGeneric) return 1;
+int bags_per_tile(int variant) {  // every variant but kVarGeneric, whose tiles follow each field's width
   const int r = kWave / lanes_of(variant);
   return kRounds * r <= kWave ? kRounds * r : kWave;  // as TileShape::NB
 }
@@ -1597,15 +1795,13 @@ constexpr int64_t kSubThresholdBinned = 48;
 constexpr int64_t kFusedSubThreshold = 48;
 
 int64_t default_sub_threshold(int variant, bool bins) {
-  if (variant == kVarGeneric) return kNoLimit;  // the element-wise kernel never splits
+  if (variant == kVarGeneric) return kNoLimit;  // the ragged kernel never splits
   return bins ? kSubThresholdBinned : kSubThreshold;
 }
 
 // With binning, bags longer than this go to the long kernel.
 constexpr int64_t kDefaultBlockThreshold = 512;
 constexpr int64_t kDefaultSplitThreshold = 192;   // listed bags longer than this are split over a workgroup
-// Longest bag pooled by one subgroup (longer ones are split over the wavefront).
-constexpr int64_t kMaxShortBag = int64_t{1} << 24;
 
 int pick_variant(const cti_ebag_table& t, int tb, int ob, const void* out, int64_t out_row_stride) {
   const int64_t row_bytes = static_cast<int64_t>(t.dim) * tb;
@@ -1696,7 +1892,7 @@ hipError_t launch_variant(int variant, const PoolParams& p, const LongList* l, h
     case kVarL64V4: launch_shape<TT, OT, 64, 4>(p, l, s); break;
     case kVarMixed: launch_mixed<TT, OT>(p, l, s); break;
     default:
-      hipLaunchKernelGGL((pool_generic_kernel<TT, OT>), dim3(static_cast<unsigned>(p.num_tiles)), dim3(kMainThreads), 0, s, p);
+      hipLaunchKernelGGL((pool_ragged_kernel<TT, OT>), dim3(static_cast<unsigned>(p.num_tiles)), dim3(kMainThreads), 0, s, p);
       break;
   }
   return hipGetLastError();
@@ -1845,6 +2041,8 @@ int run_job(const Job& j, hipStream_t stream) {
     } else {
       if (mixed && v >= kMixedLo && v <= kMixedHi && !(stream_apart && v == kVarStream)) continue;
       for (int f = 0; f < j.num_fields; ++f) if (var[f] == v) fields.push_back(f);
+      if (v == kVarGeneric)  // narrowest rows first (see pool_ragged_kernel)
+        std::stable_sort(fields.begin(), fields.end(), [&](int a, int b) { return j.tables[a].dim < j.tables[b].dim; });
     }
     for (size_t c0 = 0; c0 < fields.size(); c0 += kMaxFields) {
       PoolParams p;
@@ -1890,10 +2088,11 @@ int run_job(const Job& j, hipStream_t stream) {
         const int f = fields[c0 + i];
         const cti_ebag_table& t = j.tables[f];
         FieldDesc& d = p.f[i];
-        const int bpt = bags_per_tile(var[f]);
-        d.lanes_log2 = var[f] <= 6 ? var[f] : 0;
+        const int chunks = ragged_chunks(t.dim, tb == 1 ? 8 : 16 / tb);
+        const int bpt = v == kVarGeneric ? ragged_side(chunks) : bags_per_tile(var[f]);
+        d.lanes = v == kVarGeneric ? chunks : (var[f] <= 6 ? var[f] : 0);
         d.tile_begin = static_cast<int32_t>(tiles < INT32_MAX ? tiles : INT32_MAX);
-        tiles += (j.batch + bpt - 1) / bpt;
+        tiles += v == kVarGeneric ? ((j.batch + bpt - 1) / bpt + 7) / 8 : (j.batch + bpt - 1) / bpt;
         d.table = static_cast<const char*>(t.data);
         d.row_scale = j.tdt == CTI_EBAG_I8 ? t.row_scale : nullptr;
         d.max_row = t.rows - 1;
@@ -1906,9 +2105,14 @@ int run_job(const Job& j, hipStream_t stream) {
         // buffer path: power-of-two rows of >= 8 bytes and (rows + 1) * row_bytes <= 2^32, so the
         // pad row id 0xffffffff >> log2(row_bytes) addresses past both the rows and the scales
         const bool fits = d.row_bytes >= 8 && t.rows < (int64_t{1} << 32) / d.row_bytes;
-        d.span_bytes = pow2 && fits ? static_cast<uint32_t>(span) : 0u;
+        // the ragged kernel's buffer loads: whole chunks of 4-byte aligned rows, and no offset from the
+        // table's end on (span + a chunk's offset in the row) wraps around 32 bits
+        const bool ragged_buf = t.dim * tb >= 16 && reinterpret_cast<uintptr_t>(t.data) % 4 == 0 && d.row_bytes % 4 == 0 &&
+                                span + static_cast<int64_t>(t.dim) * tb < (int64_t{1} << 32);
+        d.span_bytes = (v == kVarGeneric ? ragged_buf : pow2 && fits) ? static_cast<uint32_t>(span) : 0u;
         all_buf = all_buf && d.span_bytes != 0;
       }
+      if (v == kVarGeneric) tiles *= 8;
       if (tiles > INT32_MAX)
         return set_error(CTI_EBAG_EUNSUPPORTED, "batch of %lld samples needs more than 2^31 tiles", (long long)j.batch);
       p.buffer_ok = all_buf ? 1 : 0;

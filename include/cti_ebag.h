@@ -310,7 +310,7 @@ int cti_ebag_fused_all_slots_typed(const void* values, int32_t index_type, const
  *                   tile holds)
  *   order           HOST int32 buffer of order_bytes >= cti_ebag_order_bytes(batch_size, num_slots)
  *   num_threads     host threads to use (1..256; the staging calls' persistent pool)
- * CTI_EBAG_EUNSUPPORTED for rows that take the element-wise kernel (not whole 16-byte vectors,
+ * CTI_EBAG_EUNSUPPORTED for rows that take the ragged kernel (not whole 16-byte vectors,
  * or wider than 4 KB) and for more than 64 slots. Synchronous.
  */
 int cti_ebag_order_host(const void* offsets, int32_t offset_type, int64_t offsets_stride, int64_t batch_size,

@@ -92,3 +92,42 @@ def test_mixed_integer_tables_exact(pkg, dev):
     for kw in BIN_SETTINGS + [dict(long_threshold=-1)]:
         got = _pool(pkg, dev, case.values, case.offsets, tables, "sum", "f32", **kw)
         assert np.array_equal(got, want), kw
+
+
+# widths around the lane vectors, the bags side by side (64 / chunks, at most 32) and the 64-chunk
+# blocks of the ragged kernel
+RAGGED = {"bf16": (1, 3, 7, 9, 10, 15, 24, 100, 168, 176, 300, 504, 520, 600, 1030),
+          "f16": (2, 8, 17, 33, 136), "f32": (1, 3, 5, 6, 50, 84, 100, 252, 260, 515), "i8": (1, 7, 9, 20, 50, 200, 513)}
+
+
+@pytest.mark.parametrize("tdt", ["bf16", "f16", "f32", "i8"])
+@pytest.mark.parametrize("B", [1, 33, 203])
+@pytest.mark.parametrize("layout", ["packed", "strided", "odd base"])
+def test_ragged_widths_match_oracle(pkg, dev, tdt, B, layout):
+    """Rows that no fixed shape holds: sums and means in element order, bit for bit, whatever the
+    bag's length, the rows' alignment and the neighbours' widths."""
+    print(f"ragged {tdt} B={B} {layout}", flush=True)
+    dims = RAGGED[tdt]
+    case = random_case(4400 + B, F=len(dims), B=B, dims=dims, V=(50, 900), tdt="f32" if tdt == "i8" else tdt, max_len=20,
+                       long_every=16, long_len=150)
+    host, tables = [], []
+    for i, t in enumerate(case.tables):
+        if tdt == "i8":
+            q = np.clip(np.rint(t * 40), -127, 127).astype(np.int8)
+            scale = (np.arange(len(q)) % 13 + 1).astype(np.float32) * np.float32(0.013)
+            host.append((q, scale))
+            w = torch.from_numpy(q).to(dev)
+        else:
+            host.append(t)
+            w = to_dev(t, tdt, dev)
+        V, D = w.shape
+        pitch, first = {"packed": (D, 0), "strided": (D + i % 5, 0), "odd base": (D, 1)}[layout]
+        flat = torch.zeros(V * pitch + first, dtype=w.dtype, device=dev)
+        view = torch.as_strided(flat, (V, D), (pitch, 1), first)
+        view.copy_(w)
+        tables.append((view, torch.from_numpy(scale).to(dev)) if tdt == "i8" else view)
+    for pooling in ("sum", "mean"):
+        for odt in ("f32", "bf16"):
+            got = _pool(pkg, dev, case.values, case.offsets, tables, pooling, odt, long_threshold=2 ** 31 - 1)
+            want = orc.pool_c(case.values, case.offsets, host, tdt, pooling, odt)
+            assert np.array_equal(got, want), (pooling, odt)
