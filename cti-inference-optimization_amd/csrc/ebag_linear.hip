@@ -10,16 +10,18 @@
 // per-row mean and rstd come from the pooling or statistics pass (cti_ebag_layernorm with no
 // output). Without statistics the kernel is the plain Linear.
 //
-// Two forms (the products on v_mfma_f32_16x16x32_bf16: lane l supplies A[l%16][8(l/16) .. +8)
+// Three forms (the products on v_mfma_f32_16x16x32_bf16: lane l supplies A[l%16][8(l/16) .. +8)
 // and B[8(l/16) .. +8)[l%16] and receives C[4(l/16) + r][l%16], r < 4; workgroups numbered so
 // that the tiles of one row band run on one XCD, whose L2 then serves the band to each of them):
-//   ln_linear_big_kernel  K a multiple of 128 (every encoder shape): 128 x 256 or 128 x 128 tiles
-//                         of 8 wavefronts, both operands through LDS (XOR-swizzled rows);
+//   ln_linear_band_kernel many rows, K a multiple of 128: bands of 128 rows by 256, 384 or 512
+//                         columns, the weight loaded straight to LDS;
+//   ln_linear_big_kernel  K a multiple of 128, fewer rows: 128 x 256 or 128 x 128 tiles of 8
+//                         wavefronts, both operands through LDS (XOR-swizzled rows);
 //   ln_linear_kernel      any K (a multiple of 8): 64 x 256 tiles of 4 wavefronts, each owning 64
 //                         columns, x through LDS and the weight's fragments straight to registers.
-// Both walk K in steps of 64 with each step's loads issued two steps ahead into rotating register
-// sets, x normalised on its way to LDS, two LDS buffers and one barrier per step. When the large
-// form's tiles would leave CUs idle (few rows), K is split over several workgroups per tile: each
+// The last two walk K in steps of 64 with each step's loads issued two steps ahead into rotating
+// register sets, x normalised on its way to LDS, two LDS buffers and one barrier per step. When the
+// tiles would leave CUs idle (few rows), K is split over several workgroups per tile: each
 // writes its fp32 partial products to a caller's workspace and ln_linear_reduce_kernel adds the
 // splits in split order, adds the bias and rounds once.
 #include <stdint.h>
@@ -56,6 +58,8 @@ struct LinearParams {
   int32_t tiles_n;
   float* part;          // split K: fp32 partial products [splits, M, N] (no bias), NULL: no split
   int32_t split_steps;  // split K: steps of kBK per split (even); split s is blockIdx.y
+  int32_t bias_f32;     // bias is fp32 (else bf16)
+  int32_t y_f32;        // y is fp32 (else bf16)
 };
 
 // One bf16 chunk (8 elements) normalised: ((x - mean) * rstd) * g + b, rounded to bf16.
@@ -268,6 +272,13 @@ __device__ __forceinline__ uint4 bload16(Rsrc r, uint32_t voff, uint32_t soff) {
   return make_uint4(v.x, v.y, v.z, v.w);
 }
 
+// 16 bytes per lane straight to LDS, lane l's to lds + 16 l (lds the same for every lane).
+__device__ __forceinline__ void bload16_lds(Rsrc r, uint4* lds, uint32_t voff, uint32_t soff) {
+#ifdef __HIP_DEVICE_COMPILE__  // the host pass has no 16-byte form
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, soff, 0, 0);
+#endif
+}
+
 // The large form (K a multiple of 128, byte offsets below 2^31): a workgroup of 8 wavefronts
 // (2 x 4, each 64 x BN/4) owns a 128 x BN tile of y (BN = 256, or 128 when that leaves fewer
 // than two tiles per CU); both
@@ -463,6 +474,278 @@ __global__ void __launch_bounds__(2 * GN * kWave, GN == 2 ? 2 : 1) ln_linear_big
   }
 }
 
+// Workgroup barrier for what the wavefronts exchanged through ds_write / ds_read: loads in flight, those
+// to LDS included, stay in flight (__syncthreads would wait for the latter).
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // no instruction: keeps the compiler's order
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+constexpr int kBandParams = 28 * 1024;  // LDS for gamma and beta (160 KB in all)
+
+// Waits until at most N of this wavefront's loads are in flight: all but the N newest have arrived, those to
+// LDS included (the compiler does not follow every load to LDS around a loop).
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | (N >> 4 << 14));  // vmcnt(N)
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The band form (K a multiple of 128, byte offsets below 2^31, gamma and beta within kBandParams): a
+// workgroup of 8 wavefronts owns 128 rows and 128 * NI columns of y, every wavefront all 128 rows of
+// 16 * NI columns of its own. So x is normalised once per band (once per element when the columns
+// cover N) on its way through registers to LDS, from where every wavefront reads it. The weight, which
+// no two wavefronts of the workgroup share, is loaded straight to LDS without passing registers, half a
+// step (32 of K) at a time into a wavefront's own two buffers, and needs no barrier: a half step first
+// waits for its weight, reads its fragments, and, once its first products have waited for those, loads
+// the next step's over them. x is loaded two steps ahead, after the step's weight loads (loads return
+// in order, so the wait for a weight must not include the newest x). One barrier per pair of steps (two
+// pairs of x buffers); fragments are read three groups of products ahead and the normalisation's vector
+// instructions go between the products. The products are taken transposed (weight as the first
+// operand), so a lane holds 4 consecutive columns of a row and stores them at once.
+// Measured, M = 30000, K = 3584, N = 512, bf16 parameters: 110-126 us (870-1000 TFLOP/s; 128 x 128 tiles:
+// 200 us). Weight fragments loaded from L2 to registers, each lane a row of its own, took 157 us (64 cache
+// lines per load instruction), 32 x 32 products 150 us, one barrier per step 133 us.
+template <int W, int NI, bool LN, typename PT>
+__global__ void __launch_bounds__(W * kWave, 2) ln_linear_band_kernel(const LinearParams p) {
+  constexpr int BM = 128, THREADS = W * kWave, BN = 16 * NI * W;
+  constexpr int MI = BM / 16;
+  constexpr int PA = BM * kChunks / THREADS;     // x chunks per thread and step
+  constexpr int kRowStep = THREADS / kChunks;
+  constexpr int HV = Elem<PT>::kBytes / 2;       // 16-byte vectors of 8 parameters
+  constexpr int PV = LN ? 2 * HV : 1;
+  static_assert(kRowStep % 8 == 0, "a thread's rows share their swizzle");
+  // rows of 128 bytes, chunk c of row r in slot c ^ (r & 7) (no bank conflicts)
+  __shared__ __align__(16) uint16_t sA[4][BM * kBK];  // two pairs of steps
+  // the weight, half a step (32 of K) at a time, by wavefront: 64-byte rows, chunk c of row r in slot
+  // c ^ (r >> 1 & 3)
+  __shared__ __align__(16) uint4 sW0[W][NI][kWave];  // first halves
+  __shared__ __align__(16) uint4 sW1[W][NI][kWave];  // second halves
+  __shared__ uint4 s_par[LN ? kBandParams / 16 : 1];  // gamma and beta of this workgroup's steps
+
+  const int tile = static_cast<int>(blockIdx.x);
+  const int64_t m0 = static_cast<int64_t>(tile / p.tiles_n) * BM;
+  const int n0 = (tile % p.tiles_n) * BN;
+  const int t = static_cast<int>(threadIdx.x);
+  const int lane = t & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(t / kWave);
+  const int kc = t % kChunks, r0 = t / kChunks;
+  const int fr = lane & 15, fq = lane >> 4;  // fragment row, 16-byte chunk of a 32-element half step
+
+  const Rsrc xr = make_rsrc(p.x, static_cast<uint32_t>(p.M * p.K * 2));
+  const Rsrc wr = make_rsrc(p.w, static_cast<uint32_t>(static_cast<int64_t>(p.N) * p.K * 2));
+  // rows past M and columns past N read the last one: their products are not stored
+  float mean[PA], rstd[PA];
+  uint32_t xoff[PA], woff[NI];
+#pragma unroll
+  for (int q = 0; q < PA; ++q) {
+    const int64_t m = m0 + r0 + q * kRowStep;
+    const int64_t mc = m < p.M ? m : p.M - 1;
+    mean[q] = 0.f;
+    rstd[q] = 1.f;
+    if constexpr (LN) {
+      mean[q] = p.mean[mc];
+      rstd[q] = p.rstd[mc];
+    }
+    xoff[q] = static_cast<uint32_t>((mc * p.K + kc * 8) * 2);
+  }
+  const int nw = n0 + wave * 16 * NI;  // the wavefront's first column
+#pragma unroll
+  for (int c = 0; c < NI; ++c) {  // lane l loads chunk (l & 3) ^ .. of row l / 4 of fragment c
+    const int n = nw + c * 16 + (lane >> 2);
+    const int chunk = (lane & 3) ^ (lane >> 3 & 3);
+    woff[c] = static_cast<uint32_t>((static_cast<int64_t>(n < p.N ? n : p.N - 1) * p.K + chunk * 8) * 2);
+  }
+
+  // this workgroup's steps of K: all of them, or split blockIdx.y's range (an even count)
+  const int nk_all = p.K / kBK;
+  const int ks0 = p.part ? static_cast<int>(blockIdx.y) * p.split_steps : 0;
+  const int nk = p.part ? (nk_all - ks0 < p.split_steps ? nk_all - ks0 : p.split_steps) : nk_all;
+
+  uint4 ra[2][PA];   // x of steps s + 1 (set (s + 1) % 2) and s + 2
+  // a step of this workgroup, the last one in place of those past it (which are never used)
+  const auto step = [&](int ks) { return static_cast<uint32_t>(ks0 + (ks < nk ? ks : nk - 1)); };
+  auto issue_x = [&](int ks, uint4 (&a)[PA]) {
+#pragma unroll
+    for (int q = 0; q < PA; ++q) a[q] = bload16(xr, xoff[q], step(ks) * kBK * 2);
+  };
+  // weight loads straight to LDS, lane l's 16 bytes to slot l
+  auto issue_w = [&](int ks, auto half) {
+    constexpr int h = decltype(half)::value;
+#pragma unroll
+    for (int c = 0; c < NI; ++c)
+      bload16_lds(wr, h ? &sW1[wave][c][0] : &sW0[wave][c][0], woff[c], step(ks) * kBK * 2 + h * 64);
+  };
+  uint4 rp[PV];  // gamma and beta of the step being normalised
+  auto read_p = [&](int ks) {
+    if constexpr (LN) {
+      const uint4* const pp = s_par + (static_cast<int>(step(ks) - ks0) * kChunks + kc) * PV;
+#pragma unroll
+      for (int h = 0; h < PV; ++h) rp[h] = pp[h];
+    }
+  };
+  auto put_x = [&](uint16_t* to, const uint4 (&a)[PA], int q0, int q1) {
+    float g[8], bt[8];
+    if constexpr (LN) {
+#pragma unroll
+      for (int h = 0; h < HV; ++h) {
+        unpack16(rp[h], g + h * (16 / Elem<PT>::kBytes), PT{});
+        unpack16(rp[HV + h], bt + h * (16 / Elem<PT>::kBytes), PT{});
+      }
+    }
+#pragma unroll
+    for (int q = q0; q < q1; ++q) {
+      uint4 v = a[q];
+      if constexpr (LN) v = normalise8(a[q], mean[q], rstd[q], g, bt);
+      *reinterpret_cast<uint4*>(to + q * kRowStep * kBK) = v;
+    }
+  };
+  f32x4 acc[MI][NI];
+#pragma unroll
+  for (int a = 0; a < MI; ++a)
+#pragma unroll
+    for (int c = 0; c < NI; ++c) acc[a][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // this thread's place in a step's x buffer: where it writes, and its fragments of either half
+  constexpr int kPair = 2 * BM * kBK;
+  uint16_t* const put_at = &sA[0][r0 * kBK + ((kc ^ (r0 & 7)) << 3)];
+  const uint16_t* const frag_at0 = &sA[0][fr * kBK + ((fq ^ (fr & 7)) << 3)];
+  const uint16_t* const frag_at1 = &sA[0][fr * kBK + (((4 + fq) ^ (fr & 7)) << 3)];
+  const int wslot = fr * 4 + (fq ^ (fr >> 1 & 3));
+  bf16x8 wb[2][NI];
+  auto read_w = [&](auto half) {
+    constexpr int h = decltype(half)::value;
+#pragma unroll
+    for (int c = 0; c < NI; ++c)
+      wb[h][c] = __builtin_bit_cast(bf16x8, h ? sW1[wave][c][wslot] : sW0[wave][c][wslot]);
+  };
+  auto multiply = [&](int i, const bf16x8& fa) {
+#pragma unroll
+    for (int c = 0; c < NI; ++c)
+      acc[i % MI][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[i / MI][c], fa, acc[i % MI][c], 0, 0, 0);
+  };
+
+  constexpr std::integral_constant<int, 0> first{};
+  constexpr std::integral_constant<int, 1> second{};
+  issue_x(0, ra[0]);
+  issue_w(0, first);
+  issue_w(0, second);
+  issue_x(1, ra[1]);
+  if constexpr (LN) {
+    // gamma and beta of this workgroup's steps, 8 of each next to one another
+    for (int i = t; i < nk * kChunks; i += THREADS) {
+      const int64_t at = (static_cast<int64_t>(ks0) * kChunks + i) * HV;
+#pragma unroll
+      for (int h = 0; h < HV; ++h) {
+        s_par[i * 2 * HV + h] = static_cast<const uint4*>(p.gamma)[at + h];
+        s_par[i * 2 * HV + HV + h] = static_cast<const uint4*>(p.beta)[at + h];
+      }
+    }
+    __syncthreads();
+  }
+  read_p(0);
+  put_x(put_at, ra[0], 0, PA);
+  issue_x(2, ra[0]);
+  read_p(1);
+  put_x(put_at + BM * kBK, ra[1], 0, PA);
+  __builtin_amdgcn_sched_barrier(0);
+  issue_x(3, ra[1]);
+  lds_barrier();
+  constexpr int kAhead = 3;  // x fragments are read this many groups of products ahead
+  // One half of step s: its fragments are read and the first products issued, which have then
+  // waited for the weight's fragments; so the next step's half may be loaded over them. Then the
+  // rest of the products, the normalisation's vector instructions between them.
+  auto half_step = [&](int u, int s, int par, auto half) {
+    constexpr int h = decltype(half)::value;
+    const uint16_t* const from = (h ? frag_at1 : frag_at0) + par * kPair + u * BM * kBK;
+    const auto frag = [&](int i) { return *reinterpret_cast<const bf16x8*>(from + i * 16 * kBK); };
+    bf16x8 fa[MI];
+    // loads issued since this half's weight: the other half's, and x (see the loop below)
+    wait_loads<NI + PA>();
+    read_w(half);
+#pragma unroll
+    for (int i = 0; i <= kAhead; ++i) fa[i] = frag(i);
+    if (h == 0) read_p(s + 2);
+    multiply(h * MI, fa[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);  // the SIMD's other wavefront reads and waits meanwhile
+    issue_w(s + 1, half);
+#pragma unroll
+    for (int i = kAhead + 1; i < MI; ++i) fa[i] = frag(i);
+#pragma unroll
+    for (int i = 1; i < MI; ++i) multiply(h * MI + i, fa[i]);
+    put_x(put_at + (par ^ 1) * kPair + u * BM * kBK, ra[u], h ? PA / 2 : 0, h ? PA : PA / 2);
+    __builtin_amdgcn_sched_group_barrier(0x20, NI, 0);
+#pragma unroll
+    for (int i = 1; i < MI; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x8, NI, 0);                        // products
+      if (i + kAhead < MI) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
+      if (LN) __builtin_amdgcn_sched_group_barrier(0x2, 12, 0);                // vector ALU
+    }
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // a pair of steps is multiplied while the next pair is normalised into the other two buffers, with
+  // one barrier per pair; nk is even
+  for (int s0 = 0, par = 0; s0 < nk; s0 += 2, par ^= 1) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      half_step(u, s0 + u, par, first);
+      half_step(u, s0 + u, par, second);
+      issue_x(s0 + u + 4, ra[u]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    lds_barrier();
+  }
+
+  // lane l holds y[m0 + 16 a + l % 16][nw + 16 c + 4 (l / 16) + r]
+  float* const part = p.part ? p.part + static_cast<int64_t>(blockIdx.y) * p.M * p.N : nullptr;
+  const bool whole = p.N % 4 == 0;  // then 4 columns starting at a multiple of 4 are all inside or all outside
+#pragma unroll
+  for (int c = 0; c < NI; ++c) {
+    const int n = nw + c * 16 + fq * 4;
+    if (n >= p.N) continue;
+    float bias[4] = {0.f, 0.f, 0.f, 0.f};
+    if (p.bias && !part) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int nr = n + r < p.N ? n + r : p.N - 1;
+        bias[r] = p.bias_f32 ? static_cast<const float*>(p.bias)[nr]
+                             : bf16_bits_to_f32(static_cast<const uint16_t*>(p.bias)[nr]);
+      }
+    }
+#pragma unroll
+    for (int a = 0; a < MI; ++a) {
+      const int64_t m = m0 + a * 16 + fr;
+      if (m >= p.M) continue;
+      const int64_t at = m * p.N + n;
+      f32x4 v = acc[a][c];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] += bias[r];
+      if (part || p.y_f32) {
+        float* const y = (part ? part : reinterpret_cast<float*>(p.y)) + at;
+        if (whole) {
+          *reinterpret_cast<f32x4*>(y) = v;
+        } else {
+          for (int r = 0; r < 4 && n + r < p.N; ++r) y[r] = v[r];
+        }
+      } else {
+        uint16_t* const y = reinterpret_cast<uint16_t*>(p.y) + at;
+        if (whole) {
+          *reinterpret_cast<u32x2*>(y) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+        } else {
+          for (int r = 0; r < 4 && n + r < p.N; ++r) y[r] = static_cast<uint16_t>(pack_bf16x2(v[r], 0.f));
+        }
+      }
+    }
+  }
+}
+
 // Split K: y[m, n] = (sum over splits, in split order, of the fp32 partials) + bias, one rounding.
 // Four consecutive elements per thread (16-byte loads of each split's partials; M * N is a
 // multiple of 4, so every split's block stays 16-byte aligned), the last thread taking the rest.
@@ -499,6 +782,26 @@ __global__ void __launch_bounds__(256) ln_linear_reduce_kernel(const LinearParam
   }
 }
 
+template <typename BT, typename OT>
+void launch_reduce(const LinearParams& p, int splits, hipStream_t s) {
+  const int64_t threads = (p.M * p.N + 3) / 4;
+  hipLaunchKernelGGL((ln_linear_reduce_kernel<BT, OT>), dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0,
+                     s, p, splits);
+}
+
+template <int NI, bool LN, typename PT, typename BT, typename OT>
+hipError_t launch_band(LinearParams p, int splits, hipStream_t s) {
+  constexpr int W = 8;
+  p.tiles_m = static_cast<int32_t>((p.M + 127) / 128);
+  p.tiles_n = (p.N + 16 * NI * W - 1) / (16 * NI * W);
+  if (splits <= 1) p.part = nullptr;
+  hipLaunchKernelGGL((ln_linear_band_kernel<W, NI, LN, PT>),
+                     dim3(static_cast<unsigned>(p.tiles_m * p.tiles_n), static_cast<unsigned>(splits > 1 ? splits : 1)),
+                     dim3(W * kWave), 0, s, p);
+  if (splits > 1) launch_reduce<BT, OT>(p, splits, s);
+  return hipGetLastError();
+}
+
 template <int BN, int GN, int U, bool LN, typename PT, typename BT, typename OT>
 hipError_t launch_big(LinearParams p, int splits, hipStream_t s) {
   p.tiles_m = static_cast<int32_t>((p.M + 127) / 128);
@@ -508,11 +811,7 @@ hipError_t launch_big(LinearParams p, int splits, hipStream_t s) {
   hipLaunchKernelGGL((ln_linear_big_kernel<BN, GN, U, LN, PT, BT, OT>),
                      dim3(static_cast<unsigned>(blocks), static_cast<unsigned>(splits > 1 ? splits : 1)),
                      dim3(2 * GN * kWave), 0, s, p);
-  if (splits > 1) {
-    const int64_t threads = (p.M * p.N + 3) / 4;
-    hipLaunchKernelGGL((ln_linear_reduce_kernel<BT, OT>), dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256),
-                       0, s, p, splits);
-  }
+  if (splits > 1) launch_reduce<BT, OT>(p, splits, s);
   return hipGetLastError();
 }
 
@@ -532,17 +831,20 @@ bool big_form(int64_t M, int32_t N, int32_t K) {
   return K % (2 * kBK) == 0 && (M + 128) * K * 2 < (int64_t{1} << 31) && static_cast<int64_t>(N) * K * 2 < (int64_t{1} << 31);
 }
 
-// Split K for the large form: enough splits that its 128 x 128 tiles give one workgroup per CU
-// (each split at least two steps of kBK, an even count), as many as `ws_bytes` of fp32 partials
-// hold; 1 = no split. `steps` receives the steps per split. (Two workgroups per CU measured
-// slower: M = 1024, K = 3584, N = 512 took 28.0 against 18.7 us, the partials' HBM traffic
-// outweighing the extra parallelism.)
-int split_count(int64_t M, int32_t N, int32_t K, int64_t ws_bytes, int* steps) {
+// Column fragments per wavefront of the band form: 8 wavefronts cover N = 256, 384 or 512 columns.
+int band_fragments(int32_t N) { return N <= 256 ? 2 : (N <= 384 ? 3 : 4); }
+
+int64_t band_tiles(int64_t M, int32_t N) {
+  const int bn = 128 * band_fragments(N);
+  return (M + 127) / 128 * ((N + bn - 1) / bn);
+}
+
+// Split K into at most `want` parts of even step counts, as many as `ws_bytes` of fp32 partials hold;
+// 1 = no split. `steps` receives the steps per split.
+int split_count(int64_t want, int64_t M, int32_t N, int32_t K, int64_t ws_bytes, int* steps) {
   const int nk = K / kBK;
   *steps = nk;
-  const int64_t tiles = (M + 127) / 128 * ((N + 127) / 128);
-  if (tiles >= kSplitTarget || nk < 4) return 1;
-  int64_t want = (kSplitTarget + tiles - 1) / tiles;
+  if (want <= 1 || nk < 4) return 1;
   const int64_t fit = ws_bytes / (M * N * 4);
   if (want > fit) want = fit;
   if (want > nk / 2) want = nk / 2;
@@ -552,15 +854,55 @@ int split_count(int64_t M, int32_t N, int32_t K, int64_t ws_bytes, int* steps) {
   return (nk + per - 1) / per;
 }
 
+// The band form where it is the fastest: from about a workgroup per CU on (its 128 x 512 tiles; narrower
+// ones from 192 tiles), and below that, with K split, where tiles times steps of K outweigh the partial
+// products (N = 384, three of the other form's 128-column tiles: a quarter of that). Measured, bf16
+// parameters, us of the 128 x 128 / 128 x 256 form against this one:
+//   K = 3584, M = 30000   N = 256 / 384 / 512: 104 / 151 / 200 against 66 / 90 / 112
+//   K = 896, M = 30000    N = 256 / 384 / 512: 34 / 50 / 64 against 24 / 33 / 42
+//   M = 16384, N = 512    K = 896 / 1792 / 3584: 33 / 55 / 101 against 33 / 51 / 84 (2 splits)
+//   M = 8192              N = 384, K = 3584: 62 against 45; N = 512, K = 7168: 96 against 82;
+//                         N = 512, K = 3584: 51 against 58 (kept with the 128 x 128 tiles)
+bool band_form(int64_t M, int32_t N, int32_t K, int param_bytes) {
+  if (!big_form(M, N, K) || static_cast<int64_t>(K) * 2 * param_bytes > kBandParams) return false;
+  const int ni = band_fragments(N);
+  const int64_t tiles = band_tiles(M, N);
+  return tiles >= (ni == 2 ? 192 : 128) || tiles * (K / kBK) >= (ni == 3 ? 1792 : 7168);
+}
+
+// The band form's K splits: as many as keep its workgroups within one per CU.
+int band_splits(int64_t M, int32_t N, int32_t K, int64_t ws_bytes, int* steps) {
+  return split_count(kSplitTarget / band_tiles(M, N), M, N, K, ws_bytes, steps);
+}
+
+// The 128 x 128 tiles' K splits: enough for one workgroup per CU. (Two per CU measured slower: M = 1024,
+// K = 3584, N = 512 took 28.0 against 18.7 us, the partials' HBM traffic outweighing the extra
+// parallelism.)
+int tile_splits(int64_t M, int32_t N, int32_t K, int64_t ws_bytes, int* steps) {
+  const int64_t tiles = (M + 127) / 128 * ((N + 127) / 128);
+  return split_count((kSplitTarget + tiles - 1) / tiles, M, N, K, ws_bytes, steps);
+}
+
 // 128 x 256 tiles when there are at least two per CU, else 128 x 128 (split over K when even
-// those leave CUs idle); the general form for the rest.
+// those leave CUs idle), where the band form does not apply; the general form for the rest.
 template <bool LN, typename PT, typename BT, typename OT>
 hipError_t launch_linear(const LinearParams& p, int64_t ws_bytes, hipStream_t s) {
+  if (band_form(p.M, p.N, p.K, LN ? Elem<PT>::kBytes : 0)) {
+    LinearParams q = p;
+    int steps = 0;
+    const int splits = p.part ? band_splits(p.M, p.N, p.K, ws_bytes, &steps) : 1;
+    q.split_steps = steps;
+    switch (band_fragments(p.N)) {
+      case 2: return launch_band<2, LN, PT, BT, OT>(q, splits, s);
+      case 3: return launch_band<3, LN, PT, BT, OT>(q, splits, s);
+      default: return launch_band<4, LN, PT, BT, OT>(q, splits, s);
+    }
+  }
   if (big_form(p.M, p.N, p.K)) {
     if ((p.M + 127) / 128 * ((p.N + 255) / 256) >= 2 * 256) return launch_big<256, 4, 2, LN, PT, BT, OT>(p, 1, s);
     LinearParams q = p;
     int steps = 0;
-    const int splits = p.part ? split_count(p.M, p.N, p.K, ws_bytes, &steps) : 1;
+    const int splits = p.part ? tile_splits(p.M, p.N, p.K, ws_bytes, &steps) : 1;
     q.split_steps = steps;
     return launch_big<128, 4, 2, LN, PT, BT, OT>(q, splits, s);
   }
@@ -585,7 +927,12 @@ using namespace cti;
 extern "C" int64_t cti_ebag_layernorm_linear_workspace_bytes(int64_t rows, int32_t cols, int32_t out_features) {
   if (rows < 1 || cols < 1 || out_features < 1 || !big_form(rows, out_features, cols)) return 0;
   int steps = 0;
-  const int splits = split_count(rows, out_features, cols, INT64_MAX, &steps);
+  // for whichever form the type of gamma and beta then selects
+  int splits = tile_splits(rows, out_features, cols, INT64_MAX, &steps);
+  if (band_form(rows, out_features, cols, 0)) {
+    const int band = band_splits(rows, out_features, cols, INT64_MAX, &steps);
+    if (band > splits || band_form(rows, out_features, cols, 4)) splits = band;
+  }
   return splits > 1 ? static_cast<int64_t>(splits) * rows * out_features * 4 : 0;
 }
 
@@ -631,6 +978,8 @@ extern "C" int cti_ebag_layernorm_linear(const void* x, int64_t rows, int32_t co
   p.M = rows;
   p.N = out_features;
   p.K = cols;
+  p.bias_f32 = bias_dtype == CTI_EBAG_F32;
+  p.y_f32 = y_dtype == CTI_EBAG_F32;
   p.part = workspace_bytes > 0 ? static_cast<float*>(workspace) : nullptr;
   hipStream_t s = static_cast<hipStream_t>(stream);
   hipError_t e;

@@ -214,3 +214,35 @@ def test_split_k_uses_as_many_splits_as_the_workspace_holds(pkg, dev):
                                               None, c.F32, y.data_ptr(), c.F32, ws.data_ptr(), ws_bytes, stream))
         torch.cuda.synchronize()
         assert torch.equal(y, want), ws_bytes
+
+
+# the band form's edges: its three column widths, tile counts beside the rule's limits, rows and columns
+# that are no whole tiles (also no multiple of 4), two column tiles, the smallest K, K split (rows from
+# 2,048 on), and parameters too large for its LDS copy
+BAND_SHAPES = [(24449, 128, 256), (24448, 256, 130), (16257, 128, 384), (16256, 384, 290), (16300, 640, 511),
+               (16385, 128, 500), (8200, 256, 700), (2048, 7168, 384), (8192, 7168, 512), (16384, 3584, 512)]
+
+
+@pytest.mark.parametrize("rows,cols,n", BAND_SHAPES)
+@pytest.mark.parametrize("pdt", [torch.bfloat16, torch.float32, None])
+def test_band_form_operands_exact(pkg, dev, rows, cols, n, pdt):
+    """Integer operands (as test_layer_norm_operands_exact): exact in any order of additions. The
+    expected result is computed on the GPU in float64, where it is exact too."""
+    print(f"band exact rows={rows} cols={cols} n={n} params={pdt}", flush=True)
+    g = torch.Generator(device="cpu").manual_seed(rows + cols + n)
+    x = torch.randint(-3, 4, (rows, cols), generator=g, dtype=torch.int8).to(dev).to(torch.bfloat16)
+    w = torch.randint(-1, 2, (n, cols), generator=g, dtype=torch.int8).to(dev).to(torch.bfloat16)
+    bias = torch.randint(-8, 9, (n,), generator=g).to(dev).to(torch.bfloat16)
+    kw, a = {}, x.double()
+    if pdt is not None:
+        mean = torch.randint(-2, 3, (rows,), generator=g).float().to(dev)
+        rstd = (1 + torch.randint(0, 2, (rows,), generator=g)).float().to(dev)
+        gamma = torch.randint(1, 3, (cols,), generator=g).to(dev).to(pdt)
+        beta = torch.randint(-4, 5, (cols,), generator=g).to(dev).to(pdt)
+        kw = dict(mean=mean, rstd=rstd, norm_weight=gamma, norm_bias=beta)
+        a = (a - mean[:, None]) * rstd[:, None] * gamma.double() + beta.double()
+    want = a @ w.double().T + bias.double()
+    for split_k in (True, False):
+        for odt in (torch.float32, torch.bfloat16):
+            got = pkg.layer_norm_linear(x, w, bias, out_dtype=odt, split_k=split_k, **kw)
+            assert torch.equal(got, want.to(odt)), (split_k, odt)
