@@ -83,6 +83,10 @@ namespace {
 //   rounds of R length-ranked bags per tile: 2 / 3 / 4 ran 41.7 / 42.5 / 42.1 us.
 constexpr int kRowsInFlight = 4;
 constexpr int kRounds = 2;
+// bags of a streamed tile of rows of 64 lane vectors (kRounds in a launch with a dispatch order, which
+// counts tiles of that many): 28 slots of 512 int8, 4,096 samples, pooled and normalised, 2 / 4 / 8 ran
+// 136 / 131 / 134 us (ranked tiles: 148)
+constexpr int kWideBags = 4;
 
 constexpr int kMainThreads = kWave;  // main kernel: one wavefront per workgroup
 constexpr int kBinThreads = 256;
@@ -160,6 +164,7 @@ struct PoolParams {
                             // reference's int8 kernel stores acc.to(bfloat16), online_best/infer.py:941)
   int32_t stream_ok;        // rows of 16 lane vectors may take streamed tiles (no binning, default
                             // short-bag limit, walks and id offsets within 32 bits)
+  int32_t wide_bags;        // bags per streamed tile of rows of 64 lane vectors
   int32_t stream_out;       // the output block is at least kStreamOutBytes: non-temporal stores
   FieldDesc f[kMaxFields];
 };
@@ -557,19 +562,44 @@ __device__ __forceinline__ void store_lane(OT* dst, const float* a) {
 
 // Streamed tiles serve rows of 16 lane vectors read with buffer loads: 256-byte rows of fp32 / bf16
 // / fp16 tables (4 bytes per lane) and 128-byte rows of int8 tables (2 bytes per lane, each row's
-// scale read with it).
+// scale read with it); and rows of 64 lane vectors (1 KB; int8: 512 bytes), one vector per lane, read
+// with buffer loads or, from tables of 4 GiB and more, with 64-bit uniform addresses. A wide row's id
+// is uniform, so its address costs no vector instruction; in rounds it cost every lane a 64-bit
+// product and the masking of each row (70 vector instructions a row in all, for 16 that unpack and
+// add). 28 slots of 512, 4,096 samples, mean length 8, pooled and normalised: 5 GB of bf16 143 -> 136 us
+// (5.2 TB/s of L2 misses), int8 148 -> 131 us.
 template <typename TT, int LANES, int VPL>
 struct StreamShape {
-  static constexpr bool ok = LANES == 16 && VPL == 1;
+  static constexpr bool wide = LANES == 64 && VPL == 1;
+  static constexpr bool ok = (LANES == 16 && VPL == 1) || wide;
   static constexpr int BPL = LANES * Elem<TT>::kVecBytes / kWave;  // bytes of a row per lane
-  static constexpr int K = 16;  // rows in flight: 16 VGPRs of row data (and 16 of scales)
+  // rows in flight: 16 VGPRs of row data, wide rows 32 (int8: 16; 16 wide rows in flight spill)
+  static constexpr int K = wide ? 8 : 16;
 };
 
-// The BPL bytes of one lane's part of a row (loaded zero-extended into 32 bits) into the
-// accumulators: fp32 / bf16 / fp16 as acc_word; int8 bytes as fma(q, s, acc) in element order.
+// The BPL bytes of one lane's part of a row.
+template <int BPL>
+struct LaneRow {
+  typedef uint32_t type;  // 2 bytes zero-extended, or 4
+};
+template <>
+struct LaneRow<8> {
+  typedef u32x2 type;
+};
+template <>
+struct LaneRow<16> {
+  typedef u32x4 type;
+};
+
+// One lane's part of a row into the accumulators: fp32 / bf16 / fp16 as acc_word; int8 bytes as
+// fma(q, s, acc) in element order.
 template <typename TT, int BPL>
-__device__ __forceinline__ void acc_lane(float* a, uint32_t w, float s) {
-  if constexpr (Quantized<TT>::value) {
+__device__ __forceinline__ void acc_lane(float* a, const typename LaneRow<BPL>::type& w, float s) {
+  if constexpr (BPL == 16) {
+    acc16(a, make_uint4(w.x, w.y, w.z, w.w), TT{});
+  } else if constexpr (BPL == 8) {
+    acc_row<TT>(a, make_uint4(w.x, w.y, 0u, 0u), s);
+  } else if constexpr (Quantized<TT>::value) {
 #pragma unroll
     for (int k = 0; k < BPL; ++k)
       a[k] = __builtin_fmaf(static_cast<float>(static_cast<int8_t>(w >> (8 * k))), s, a[k]);
@@ -579,9 +609,34 @@ __device__ __forceinline__ void acc_lane(float* a, uint32_t w, float s) {
   }
 }
 template <int BPL>
-__device__ __forceinline__ uint32_t load_lane(Rsrc r, unsigned int off) {
+__device__ __forceinline__ typename LaneRow<BPL>::type load_lane(Rsrc r, unsigned int off) {
   if constexpr (BPL == 2) return static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0));
-  else return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
+  else if constexpr (BPL == 4) return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
+  else if constexpr (BPL == 8) return __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
+  else return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+}
+
+// The table of a walk: read through buffers over the rows and scales (span < 4 GiB, power-of-two
+// rows; a row's handle is its byte offset), or with 64-bit addresses (its handle is its number).
+struct WalkTable {
+  Rsrc rsrc, srsrc;
+  unsigned int shift;  // log2 of the row stride (buffers)
+  const char* table;
+  const float* row_scale;
+  int64_t row_bytes;
+  int64_t max_row;
+};
+__device__ __forceinline__ WalkTable walk_table(const FieldDesc& f, bool quantized, bool buffers) {
+  WalkTable t;
+  t.rsrc = make_rsrc(f.table, buffers ? f.span_bytes : 0u);
+  t.srsrc = make_rsrc(reinterpret_cast<const char*>(f.row_scale),
+                      quantized && buffers ? static_cast<uint32_t>((f.max_row + 1) * 4) : 0u);
+  t.shift = static_cast<unsigned int>(__builtin_ctzll(static_cast<unsigned long long>(f.row_bytes)));
+  t.table = f.table;
+  t.row_scale = f.row_scale;
+  t.row_bytes = f.row_bytes;
+  t.max_row = f.max_row;
+  return t;
 }
 
 // Raw ids of one 64-row chunk (one per lane), as loaded: converted only when the chunk is used,
@@ -603,14 +658,17 @@ struct RawIds<int64_t> {
 };
 
 // Walks the rows of nb <= NB bags in order, bag after bag: lane i < nb describes bag i, the rows
-// values[start, end). Each lane holds 4 bytes of every 256-byte row (read through `rsrc`, `shift`
-// = log2 of the row stride); K row loads stay in flight across bag boundaries. When the last row
-// of bag i has been added (at once for an empty bag) it calls store(i, r) with the bag's
-// E = 4 / sizeof(TT) results of this lane (divided by the length for mean pooling), i rising.
-// Walk rows are counted in 32 bits: the bags hold fewer than 2^31 rows in all (host).
-template <typename TT, typename IT, int K, int NB, int BPL, typename Store>
-__device__ __forceinline__ void stream_walk(const PoolParams& p, Rsrc rsrc, Rsrc srsrc, unsigned int shift,
-                                            int64_t max_row, int nb, int64_t start, int64_t end, Store&& store) {
+// values[start, end). Each lane holds BPL bytes of every row; K row loads stay in flight across bag
+// boundaries. When the last row of bag i has been added (at once for an empty bag) it calls
+// store(i, r) with the bag's E = BPL / sizeof(TT) results of this lane (divided by the length for mean
+// pooling), i rising. Rows are read through buffers (BUF), or at uniform 64-bit addresses. Walk rows
+// are counted in 32 bits: the bags hold fewer than 2^31 rows in all (host).
+template <typename TT, typename IT, int K, int NB, int BPL, bool BUF, typename Store>
+__device__ __forceinline__ void stream_walk(const PoolParams& p, const WalkTable& wt, int nb, int64_t start,
+                                            int64_t end, Store&& store) {
+  const Rsrc rsrc = wt.rsrc, srsrc = wt.srsrc;
+  const unsigned int shift = wt.shift;
+  const int64_t max_row = wt.max_row;
   static_assert(kWave % K == 0 && K <= kWave, "K divides the 64-row id chunk");
   static_assert(NB <= kWave, "one lane per bag");
   constexpr bool Q = Quantized<TT>::value;
@@ -672,8 +730,21 @@ __device__ __forceinline__ void stream_walk(const PoolParams& p, Rsrc rsrc, Rsrc
     raw.load(vrsrc, t < T && at < p.nnz ? static_cast<unsigned int>(at * static_cast<int64_t>(sizeof(IT))) : 0xffffffffu);
   };
 
-  const unsigned int r_pad = 0xffffffffu >> shift;  // offsets past the table: zeros, no request
+  // past the walk: offsets past the table (zeros, no request), or row 0; never added
+  const unsigned int r_pad = BUF ? 0xffffffffu >> shift : 0u;
   const unsigned int lane_off = static_cast<unsigned int>(lane * BPL);
+  const auto row_handle = [&](int64_t id, bool live) {
+    const unsigned int r = live ? static_cast<unsigned int>(clamp_i64(id, 0, max_row)) : r_pad;
+    return BUF ? r << shift : r;
+  };
+  const auto load_row = [&](unsigned int handle) {  // of a uniform handle
+    if constexpr (BUF) {
+      return load_lane<BPL>(rsrc, handle + lane_off);
+    } else {
+      const char* const row = wt.table + static_cast<uint64_t>(handle) * static_cast<uint64_t>(wt.row_bytes);
+      return *reinterpret_cast<const typename LaneRow<BPL>::type*>(row + lane_off);
+    }
+  };
   // int8 rows: a row's scale offset is its row offset >> (shift - 2) (past the scales for the pad
   // rows, whose row offsets lie past the table: the host admits only (rows + 1) * row_bytes <= 2^32)
   const unsigned int sshift = shift - 2;
@@ -682,22 +753,26 @@ __device__ __forceinline__ void stream_walk(const PoolParams& p, Rsrc rsrc, Rsrc
   RawIds<IT> raw, raw_next;
   load_chunk(raw, 0);
   load_chunk(raw_next, kWave);
-  unsigned int ids = (lane < T ? static_cast<unsigned int>(clamp_i64(raw.value(), 0, max_row)) : r_pad) << shift;
+  unsigned int ids = row_handle(raw.value(), lane < T);
   // int8 rows: the scales of a chunk's rows, one per lane, loaded when the chunk's ids are taken
   // (pad rows read zeros past the scales); a row's scale is read with readlane when it is added.
   // sc_issue: the chunk being issued; sc_add: the chunk of the rows being added (the previous
   // one for a step, after the issue has moved on to a new chunk)
   float sc_issue = 0.f, sc_add = 0.f;
+  const auto load_scale = [&]() {
+    if constexpr (BUF) return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(srsrc, ids >> sshift, 0, 0));
+    else return wt.row_scale[ids];
+  };
   if constexpr (Q) {
-    sc_issue = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(srsrc, ids >> sshift, 0, 0));
+    sc_issue = load_scale();
     sc_add = sc_issue;
   }
 
-  uint32_t v[K];
+  typename LaneRow<BPL>::type v[K];
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const unsigned int r = static_cast<unsigned int>(__builtin_amdgcn_readlane(static_cast<int>(ids), k));
-    v[k] = load_lane<BPL>(rsrc, r + lane_off);
+    v[k] = load_row(r);
   }
 
   float acc[E];
@@ -742,9 +817,9 @@ __device__ __forceinline__ void stream_walk(const PoolParams& p, Rsrc rsrc, Rsrc
     }
     if (c_issue == 0) {
       // rows j + K .. are in the next chunk: take it, and load the one after it
-      ids = (j + K + lane < T ? static_cast<unsigned int>(clamp_i64(raw_next.value(), 0, max_row)) : r_pad) << shift;
+      ids = row_handle(raw_next.value(), j + K + lane < T);
       load_chunk(raw_next, j + K + kWave);
-      if constexpr (Q) sc_issue = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(srsrc, ids >> sshift, 0, 0));
+      if constexpr (Q) sc_issue = load_scale();
     }
     int dn = next_end - j - 1;  // step row after which the next bag ends
     unsigned int roff[K];       // this step's row offsets, uniform (scalar registers)
@@ -760,7 +835,7 @@ __device__ __forceinline__ void stream_walk(const PoolParams& p, Rsrc rsrc, Rsrc
         flush(j + k + 1);
         dn = next_end - j - 1;
       }
-      v[k] = load_lane<BPL>(rsrc, roff[k] + lane_off);
+      v[k] = load_row(roff[k]);
     }
   }
   if (j < T) {  // the partial last step: rows j .. T - 1, nothing issued
@@ -785,24 +860,23 @@ __device__ __forceinline__ void stream_walk(const PoolParams& p, Rsrc rsrc, Rsrc
 }
 
 // A tile of NB consecutive bags of one field, streamed (see stream_walk); STREAM_OUT: the results
-// are stored non-temporally (the host sets it for output blocks of kStreamOutBytes and more).
-template <typename TT, typename OT, typename IT, int K, int NB, int BPL, bool STREAM_OUT>
+// are stored non-temporally (the host sets it for output blocks of kStreamOutBytes and more; wide
+// rows, whose stores are whole vectors, decide at run time).
+template <typename TT, typename OT, typename IT, int K, int NB, int BPL, bool BUF, bool STREAM_OUT>
 __device__ __forceinline__ void pool_tile_stream(const PoolParams& p, int fi, int local_tile) {
   constexpr int E = BPL / Elem<TT>::kBytes;
   const int lane = lane_id();
-  const int64_t b0 = static_cast<int64_t>(local_tile) * NB;
-  const int nb = static_cast<int>(p.batch - b0 < NB ? p.batch - b0 : NB);
+  const int bags = E > 2 ? p.wide_bags : NB;  // at most NB
+  const int64_t b0 = static_cast<int64_t>(local_tile) * bags;
+  const int nb = static_cast<int>(p.batch - b0 < bags ? p.batch - b0 : bags);
   int64_t start = 0, end = 0;
   if (lane < nb) bag_range(p, p.f[fi].gidx, b0 + lane, start, end);
-  const Rsrc rsrc = make_rsrc(p.f[fi].table, p.f[fi].span_bytes);
-  const Rsrc srsrc = make_rsrc(reinterpret_cast<const char*>(p.f[fi].row_scale),
-                               Quantized<TT>::value ? static_cast<uint32_t>((p.f[fi].max_row + 1) * 4) : 0u);
-  const unsigned int shift =
-      static_cast<unsigned int>(__builtin_ctzll(static_cast<unsigned long long>(p.f[fi].row_bytes)));
   // bags are stored in order, each once: the destination advances by one output row per bag
   OT* dst = reinterpret_cast<OT*>(p.out) + b0 * p.out_row_stride + p.f[fi].out_col + lane * E;
-  stream_walk<TT, IT, K, NB, BPL>(p, rsrc, srsrc, shift, p.f[fi].max_row, nb, start, end, [&](int, const float* r) {
-    store_lane<OT, E, STREAM_OUT>(dst, r);
+  stream_walk<TT, IT, K, NB, BPL, BUF>(p, walk_table(p.f[fi], Quantized<TT>::value, BUF), nb, start, end,
+                                       [&](int, const float* r) {
+    if constexpr (E > 2) store_out<E>(dst, r, p.stream_out);
+    else store_lane<OT, E, STREAM_OUT>(dst, r);
     dst += p.out_row_stride;
   });
 }
@@ -967,11 +1041,12 @@ __global__ void __launch_bounds__(kMainThreads) pool_kernel(const PoolParams p) 
   const int fi = field_of_tile(p, tile);
   if constexpr (FORM != kTileRanked) {
     using Stream = StreamShape<TT, LANES, VPL>;
-    static_assert(BUF && Stream::ok, "streamed tiles need buffer loads and rows of 16 lane vectors");
+    static_assert(Stream::ok && (BUF || Stream::wide), "a streamed row shape, read with buffer loads unless wide");
     using IT = typename std::conditional<FORM == kTileStream32 || FORM == kTileStream32Nt, int32_t, int64_t>::type;
     constexpr bool kNt = FORM == kTileStream32Nt || FORM == kTileStream64Nt;
-    pool_tile_stream<TT, OT, IT, Stream::K, TileShape<TT, LANES, VPL>::NB, Stream::BPL, kNt>(p, fi,
-                                                                                           tile - fi * p.tiles_per_field);
+    constexpr int NB = Stream::wide ? kWideBags : TileShape<TT, LANES, VPL>::NB;
+    pool_tile_stream<TT, OT, IT, Stream::K, NB, Stream::BPL, BUF, kNt>(
+        p, fi, tile - fi * p.tiles_per_field);
   } else {
     pool_tile<TT, OT, LANES, VPL, BUF>(p, fi, tile - fi * p.tiles_per_field, s.tile);
   }
@@ -1039,7 +1114,9 @@ struct FusedNorm {
 // wavefronts of a fused workgroup pool independently, so no workgroup barrier is used here.
 __device__ __forceinline__ void wave_sync() { __builtin_amdgcn_wave_barrier(); }
 
-template <typename TT, typename PT, int LANES, int SPW, bool BUF, int W = fused_waves(LANES)>
+// WALK (rows of 64 lane vectors): a wavefront streams its bags' rows as the main kernel streams a tile
+// (stream_walk: uniform row addresses, K rows in flight across bags) instead of pooling them in rounds.
+template <typename TT, typename PT, int LANES, int SPW, bool BUF, bool WALK, int W = fused_waves(LANES)>
 __global__ void __launch_bounds__(W * kWave) pool_norm_kernel(const PoolParams p, const FusedNorm fn) {
   using S = Shape<TT, LANES, 1>;
   constexpr int U = S::U;
@@ -1092,6 +1169,22 @@ __global__ void __launch_bounds__(W * kWave) pool_norm_kernel(const PoolParams p
   }
   const int rd = rank / W, rm = rank - rd * W;
   const bool mine = valid && ((rd & 1) ? W - 1 - rm : rm) == wave;
+  if constexpr (WALK) {
+    static_assert(LANES == kWave, "one row per wavefront and load");
+    using Stream = StreamShape<TT, LANES, 1>;
+    constexpr int NB = kFusedBags / W;
+    if (mine) s.order[rd] = lane;
+    wave_sync();
+    const int n_mine = __popcll(__ballot(mine));
+    const int bag = lane < n_mine ? s.order[lane] : 0;  // lane i: this wavefront's i-th bag
+    const int64_t bs = shfl_i64(start, bag), be = shfl_i64(end, bag);
+    const WalkTable wt = walk_table(p.f[0], false, BUF);
+    const auto write_bag = [&](int i, const float* r) {
+      store_out<S::VEC>(row + static_cast<int64_t>(__builtin_amdgcn_readlane(bag, i)) * D + lane * S::VEC, r, false);
+    };
+    if (p.idx32) stream_walk<TT, int32_t, Stream::K, NB, Stream::BPL, BUF>(p, wt, n_mine, bs, be, write_bag);
+    else stream_walk<TT, int64_t, Stream::K, NB, Stream::BPL, BUF>(p, wt, n_mine, bs, be, write_bag);
+  } else {
   const bool medium = mine && L > p.sub_threshold;
   const bool shortb = mine && L <= p.sub_threshold;
   const int n_medium = __popcll(__ballot(medium));
@@ -1161,6 +1254,7 @@ __global__ void __launch_bounds__(W * kWave) pool_norm_kernel(const PoolParams p
     wave_sync();
     wave_slice_partial<TT, LANES, 1>(p, table, nullptr, max_row, row_bytes, bs, be, pa, s.ids);
     if (g == 0) write_row(src, be - bs, pa);
+  }
   }
   __syncthreads();  // the whole rows are in LDS
 
@@ -1841,16 +1935,22 @@ void launch_shape(const PoolParams& p, const LongList* l, hipStream_t s) {
   if (l) launch_bins(p, *l, s);
   const dim3 grid(static_cast<unsigned>(p.num_tiles) + (p.next_order ? static_cast<unsigned>(p.order_blocks) : 0u)),
       block(kMainThreads);
-  constexpr bool kStream = StreamShape<TT, LANES, VPL>::ok;
-  const bool stream = kStream && p.stream_ok && p.buffer_ok;
-  if (stream && p.idx32 && p.stream_out)
-    hipLaunchKernelGGL((pool_kernel<TT, OT, LANES, VPL, true, kStream ? kTileStream32Nt : kTileRanked>), grid, block, 0, s, p);
+  constexpr bool kStream = StreamShape<TT, LANES, VPL>::ok, kWide = StreamShape<TT, LANES, VPL>::wide;
+  constexpr bool kNt = kStream && !kWide;  // wide rows: plain and non-temporal stores in one kernel
+  const bool stream = kStream && p.stream_ok && (kWide || p.buffer_ok);
+  constexpr int kS32 = kStream ? kTileStream32 : kTileRanked, kS64 = kStream ? kTileStream64 : kTileRanked;
+  if (stream && kWide && !p.buffer_ok && p.idx32)
+    hipLaunchKernelGGL((pool_kernel<TT, OT, LANES, VPL, !kWide, kS32>), grid, block, 0, s, p);
+  else if (stream && kWide && !p.buffer_ok)
+    hipLaunchKernelGGL((pool_kernel<TT, OT, LANES, VPL, !kWide, kS64>), grid, block, 0, s, p);
+  else if (stream && p.idx32 && p.stream_out && kNt)
+    hipLaunchKernelGGL((pool_kernel<TT, OT, LANES, VPL, true, kNt ? kTileStream32Nt : kS32>), grid, block, 0, s, p);
   else if (stream && p.idx32)
-    hipLaunchKernelGGL((pool_kernel<TT, OT, LANES, VPL, true, kStream ? kTileStream32 : kTileRanked>), grid, block, 0, s, p);
-  else if (stream && p.stream_out)
-    hipLaunchKernelGGL((pool_kernel<TT, OT, LANES, VPL, true, kStream ? kTileStream64Nt : kTileRanked>), grid, block, 0, s, p);
+    hipLaunchKernelGGL((pool_kernel<TT, OT, LANES, VPL, true, kS32>), grid, block, 0, s, p);
+  else if (stream && p.stream_out && kNt)
+    hipLaunchKernelGGL((pool_kernel<TT, OT, LANES, VPL, true, kNt ? kTileStream64Nt : kS64>), grid, block, 0, s, p);
   else if (stream)
-    hipLaunchKernelGGL((pool_kernel<TT, OT, LANES, VPL, true, kStream ? kTileStream64 : kTileRanked>), grid, block, 0, s, p);
+    hipLaunchKernelGGL((pool_kernel<TT, OT, LANES, VPL, true, kS64>), grid, block, 0, s, p);
   else if (p.buffer_ok)
     hipLaunchKernelGGL((pool_kernel<TT, OT, LANES, VPL, true, kTileRanked>), grid, block, 0, s, p);
   else
@@ -1965,6 +2065,7 @@ int64_t workspace_bytes(int64_t batch, int32_t num_fields);
 // The variant whose rows are 16 lane vectors (256 bytes of fp32 / bf16 / fp16, 128 bytes of int8):
 // the streamed tiles' shape.
 constexpr int kVarStream = 4;
+constexpr int kVarWide = 6;  // rows of 64 lane vectors, streamed too
 static_assert(StreamShape<float, 1 << kVarStream, 1>::ok && StreamShape<bf16_t, 1 << kVarStream, 1>::ok &&
                   StreamShape<f16_t, 1 << kVarStream, 1>::ok && StreamShape<i8_t, 1 << kVarStream, 1>::ok &&
                   TileShape<bf16_t, 1 << kVarStream, 1>::NB == kRounds * (kWave / 16),
@@ -1973,9 +2074,13 @@ static_assert(StreamShape<float, 1 << kVarStream, 1>::ok && StreamShape<bf16_t, 
 // Whether a job's fields of the streamed shape may take streamed tiles (launch_shape also needs
 // buffer loads over every table of their launch): no binning, the default short-bag limit, and
 // walks / id offsets that fit 32 bits.
+bool stream_ids_ok(int64_t nnz, int idx32) {
+  constexpr int64_t nb = 8;  // bags per walk, each of which may hold every id (overlapping bags)
+  static_assert(kRounds * (kWave / 16) <= nb && kWideBags <= nb && kFusedBags / fused_waves(kWave) <= nb, "bags per walk");
+  return nnz < INT32_MAX / nb && nnz * (idx32 ? 4 : 8) < (int64_t{1} << 32);
+}
 bool stream_variant_allowed(const Job& j) {
-  const int64_t nb = kRounds * (kWave / 16);  // bags per tile of the streamed shape
-  return !j.use_bins && j.sub_threshold == 0 && j.nnz < INT32_MAX / nb && j.nnz * (j.idx32 ? 4 : 8) < (int64_t{1} << 32);
+  return !j.use_bins && j.sub_threshold == 0 && stream_ids_ok(j.nnz, j.idx32);
 }
 
 int run_job(const Job& j, hipStream_t stream) {
@@ -2082,6 +2187,7 @@ int run_job(const Job& j, hipStream_t stream) {
       }
       const size_t nf = fields.size() - c0 < static_cast<size_t>(kMaxFields) ? fields.size() - c0 : kMaxFields;
       p.num_fields = static_cast<int32_t>(nf);
+      p.wide_bags = p.stream_ok && !ordered ? kWideBags : bags_per_tile(kVarWide);
       bool all_buf = true;
       int64_t tiles = 0;
       for (size_t i = 0; i < nf; ++i) {
@@ -2089,7 +2195,7 @@ int run_job(const Job& j, hipStream_t stream) {
         const cti_ebag_table& t = j.tables[f];
         FieldDesc& d = p.f[i];
         const int chunks = ragged_chunks(t.dim, tb == 1 ? 8 : 16 / tb);
-        const int bpt = v == kVarGeneric ? ragged_side(chunks) : bags_per_tile(var[f]);
+        const int bpt = v == kVarGeneric ? ragged_side(chunks) : (v == kVarWide ? p.wide_bags : bags_per_tile(var[f]));
         d.lanes = v == kVarGeneric ? chunks : (var[f] <= 6 ? var[f] : 0);
         d.tile_begin = static_cast<int32_t>(tiles < INT32_MAX ? tiles : INT32_MAX);
         tiles += v == kVarGeneric ? ((j.batch + bpt - 1) / bpt + 7) / 8 : (j.batch + bpt - 1) / bpt;
@@ -2210,13 +2316,21 @@ template <typename TT, typename PT, int LANES>
 hipError_t launch_fused(const PoolParams& p, const FusedNorm& fn, int spw, size_t row_lds, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>((p.batch + spw - 1) / spw)), block(fused_waves(LANES) * kWave);
   const size_t lds = row_lds * spw;
+  constexpr bool kWalk = LANES == kWave;
+  if (kWalk && p.stream_ok) {
+    switch (spw * 2 + (p.buffer_ok ? 1 : 0)) {
+      case 2: hipLaunchKernelGGL((pool_norm_kernel<TT, PT, LANES, 1, false, kWalk>), grid, block, lds, s, p, fn); break;
+      case 3: hipLaunchKernelGGL((pool_norm_kernel<TT, PT, LANES, 1, true, kWalk>), grid, block, lds, s, p, fn); break;
+      case 4: hipLaunchKernelGGL((pool_norm_kernel<TT, PT, LANES, 2, false, kWalk>), grid, block, lds, s, p, fn); break;
+      default: hipLaunchKernelGGL((pool_norm_kernel<TT, PT, LANES, 2, true, kWalk>), grid, block, lds, s, p, fn); break;
+    }
+    return hipGetLastError();
+  }
   switch (spw * 2 + (p.buffer_ok ? 1 : 0)) {
-    case 2: hipLaunchKernelGGL((pool_norm_kernel<TT, PT, LANES, 1, false>), grid, block, lds, s, p, fn); break;
-    case 3: hipLaunchKernelGGL((pool_norm_kernel<TT, PT, LANES, 1, true>), grid, block, lds, s, p, fn); break;
-    case 4: hipLaunchKernelGGL((pool_norm_kernel<TT, PT, LANES, 2, false>), grid, block, lds, s, p, fn); break;
-    case 5: hipLaunchKernelGGL((pool_norm_kernel<TT, PT, LANES, 2, true>), grid, block, lds, s, p, fn); break;
-    case 8: hipLaunchKernelGGL((pool_norm_kernel<TT, PT, LANES, 4, false>), grid, block, lds, s, p, fn); break;
-    default: hipLaunchKernelGGL((pool_norm_kernel<TT, PT, LANES, 4, true>), grid, block, lds, s, p, fn); break;
+    case 2: hipLaunchKernelGGL((pool_norm_kernel<TT, PT, LANES, 1, false, false>), grid, block, lds, s, p, fn); break;
+    case 3: hipLaunchKernelGGL((pool_norm_kernel<TT, PT, LANES, 1, true, false>), grid, block, lds, s, p, fn); break;
+    case 4: hipLaunchKernelGGL((pool_norm_kernel<TT, PT, LANES, 2, false, false>), grid, block, lds, s, p, fn); break;
+    default: hipLaunchKernelGGL((pool_norm_kernel<TT, PT, LANES, 2, true, false>), grid, block, lds, s, p, fn); break;
   }
   return hipGetLastError();
 }
@@ -2234,6 +2348,7 @@ hipError_t launch_fused_lanes(int lanes, const PoolParams& p, const FusedNorm& f
 }
 
 constexpr int kFusedSamples = 2;  // measured: 1 / 2 / 4 samples per workgroup 45.7 / 40.5 / 44.6 us
+static_assert(kFusedSamples <= 2, "launch_fused instantiates one and two");
 
 // Samples per fused workgroup: up to kFusedSamples, while the workgroup's bags fit one lane each
 // and the LDS rows stay within kFusedLdsMax.
@@ -2306,6 +2421,7 @@ extern "C" int cti_ebag_fused_all_slots_layernorm(const void* values, int32_t in
   p.num_fields = num_slots;
   p.stream_out = batch_size * p.out_row_stride * tb >= kStreamOutBytes;
   p.sub_threshold = kFusedSubThreshold;
+  p.stream_ok = stream_ids_ok(nnz, p.idx32);
   p.block_threshold = kNoLimit;
   p.split_threshold = kNoLimit;
   const int64_t rows = max_idx + 1;

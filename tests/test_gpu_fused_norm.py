@@ -169,3 +169,83 @@ def test_encoder_normalized_uses_fused_path(pkg, dev):
     torch.cuda.synchronize()
     check(y, expected(v, ro, vo, enc.emb.weight.detach(), enc.input_norm.weight.detach(),
                       enc.input_norm.bias.detach(), B, "sum", "bf16"), "bf16")
+
+
+# rows of 64 lane vectors are streamed: tiles of 4 bags (2 with a dispatch order), tables read through
+# buffers below 4 GiB and with power-of-two rows, else at 64-bit addresses
+@pytest.mark.parametrize("tdt", ["bf16", "f32", "f16", "i8"])
+@pytest.mark.parametrize("B", [1, 4, 5, 67])
+@pytest.mark.parametrize("padded", [False, True])
+def test_wide_rows_match_oracle(pkg, dev, tdt, B, padded):
+    print(f"wide rows {tdt} B={B} padded={padded}", flush=True)
+    D = 256 if tdt == "f32" else 512
+    rng = np.random.default_rng(B)
+    F, V = 3, 200
+    L = rng.integers(0, 12, (F, B))
+    L[:, ::4] = rng.choice([0, 63, 64, 65, 130], L[:, ::4].shape)
+    off = np.concatenate([[0], np.cumsum(L.reshape(-1))]).astype(np.int64)
+    ids = rng.integers(-3, V + 3, int(off[-1])).astype(np.int64)
+    host, tables = [], []
+    for f in range(F):
+        if tdt == "i8":
+            q = rng.integers(-128, 128, (V, D)).astype(np.int8)
+            scale = (rng.random(V) * 0.02 + 1e-4).astype(np.float32)
+            host.append((q, scale))
+            t = torch.from_numpy(q).to(dev)
+        else:
+            host.append(orc.encode(rng.standard_normal((V, D)).astype(np.float32), tdt))
+            t = torch.from_numpy(host[-1].view(np.int16) if tdt != "f32" else host[-1]).to(dev)
+            t = t if tdt == "f32" else t.view(torch.bfloat16 if tdt == "bf16" else torch.float16)
+        if padded:  # rows 16 bytes apart more than their width
+            wide = torch.zeros(V, D + 16 // t.element_size(), dtype=t.dtype, device=dev)
+            wide[:, :D] = t
+            t = wide[:, :D]
+        tables.append((t, torch.from_numpy(scale).to(dev)) if tdt == "i8" else t)
+    for idt in (torch.int64, torch.int32):
+        for pooling in ("sum", "mean"):
+            got = pkg.embedding_bag_pooled(torch.from_numpy(ids).to(dev).to(idt), torch.from_numpy(off).to(dev), tables,
+                                           pooling=pooling, out_dtype=torch.float32).cpu().numpy()
+            want = orc.pool_c(ids, off, host, tdt, pooling, "f32")
+            assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (idt, pooling)
+
+
+@pytest.mark.parametrize("int8", [False, True])
+def test_wide_table_beyond_4_gib(pkg, dev, int8):
+    """A table of 4.4 GB (rows at 64-bit addresses) gives what a small table of the same rows gives
+    (rows through buffers), pooled and pooled with the LayerNorm, bit for bit."""
+    S, B, D = 28, 37, 512
+    V = 8_600_000 if int8 else 4_300_000
+    g = torch.Generator(device="cpu").manual_seed(5)
+    lens = torch.randint(0, 15, (S, B), generator=g)
+    rows = torch.zeros(S, B + 1, dtype=torch.int64)
+    rows[:, 1:] = torch.cumsum(lens, 1)
+    starts = torch.cumsum(rows[:, -1], 0) - rows[:, -1]
+    n = int(lens.sum())
+    ids = torch.randint(0, V, (n,), generator=g)
+    ids[::7] = V - 1 - ids[::7] % 100
+    uniq, small_ids = torch.unique(ids, return_inverse=True)
+    out = {}
+    with torch.device("meta"):
+        encs = {"big": pkg.RepEncoder(V, D, slot_num=S, d_model=8), "small": pkg.RepEncoder(len(uniq), D, slot_num=S, d_model=8)}
+    gamma = (1 + 0.1 * torch.randn(S * D, generator=g)).to(dev).to(torch.bfloat16)
+    beta = (0.1 * torch.randn(S * D, generator=g)).to(dev).to(torch.bfloat16)
+    if int8:
+        big = torch.randint(-128, 128, (V, D), dtype=torch.int8, device=dev)
+        scale = torch.rand(V, device=dev) * 0.01 + 1e-4
+    else:
+        big = torch.empty(V, D, dtype=torch.bfloat16, device=dev).normal_()
+    for name, enc in encs.items():
+        sel = slice(None) if name == "big" else uniq.to(dev)
+        enc.input_norm.weight = torch.nn.Parameter(gamma, requires_grad=False)
+        enc.input_norm.bias = torch.nn.Parameter(beta, requires_grad=False)
+        if int8:
+            weight = torch.empty(1, D, dtype=torch.bfloat16, device=dev).expand(enc.emb.num_embeddings, D)
+            enc._int8_weight, enc._int8_scale = big[sel].contiguous(), scale[sel].contiguous()
+        else:
+            weight = big[sel]
+        enc.emb.weight = torch.nn.Parameter(weight, requires_grad=False)
+        batch = {"_flat_values": (ids if name == "big" else small_ids).to(dev),
+                 "_flat_row_offsets": rows.reshape(-1).to(dev), "_val_offsets": starts.to(dev)}
+        out[name] = (enc.pooled(batch), enc.normalized(batch))
+    for a, b in zip(out["big"], out["small"]):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
