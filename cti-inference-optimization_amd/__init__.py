@@ -6,6 +6,7 @@ Public surface:
   fused_all_slots_embedding_layernorm   the fused step with the input LayerNorm in one kernel
   quantize_embedding_int8    int8 row quantisation of a table (int8 rows + fp32 row scales)
   fused_all_slots_embedding_int8   drop-in for the reference's int8 fused kernel launch
+  fused_all_slots_embedding_int8_layernorm   it and the input LayerNorm, in one launch for 512-wide rows
   embedding_bag_pooled       per-field tables, global offsets, sum/mean, chosen output dtype
   PooledEmbedding            the same with the table descriptors prepared once (serving loops)
   layer_norm                 the encoder's input LayerNorm over the pooled rows
@@ -24,7 +25,7 @@ from .encoder import RepEncoder
 from .layout import collate_flat_layout, merge_batches, pack_slots, prebuild_flat_layout
 from .staging import InputStager, move_model_inputs_to_device
 from .ops import (PooledEmbedding, embedding_bag_pooled, fused_all_slots_embedding, fused_all_slots_embedding_int8,
-                  fused_all_slots_embedding_layernorm, fused_embedding, layer_norm, layer_norm_linear,
+                  fused_all_slots_embedding_int8_layernorm, fused_all_slots_embedding_layernorm, fused_embedding, layer_norm, layer_norm_linear,
                   layer_norm_stats, make_tile_order, order_bytes, quantize_embedding_int8)
 
 __all__ = [
@@ -42,6 +43,7 @@ __all__ = [
     "fused_all_slots_embedding",
     "fused_embedding",
     "fused_all_slots_embedding_int8",
+    "fused_all_slots_embedding_int8_layernorm",
     "fused_all_slots_embedding_layernorm",
     "quantize_embedding_int8",
     "layer_norm",

@@ -122,6 +122,10 @@ SIGNATURES = {
         ctypes.c_int,
         [_P, _I32, _P, _P, _I32, _P, _I32, _P, _I64, _I32, _I32, _I64, _I64, _I32, _P, _P, _I32, ctypes.c_float, _P],
     ),
+    "cti_ebag_fused_all_slots_layernorm_int8": (
+        ctypes.c_int,
+        [_P, _I32, _P, _P, _I32, _P, _P, _P, _I32, _I64, _I32, _I32, _I64, _I64, _I32, _P, _P, _I32, ctypes.c_float, _P],
+    ),
     "cti_ebag_stage_copy": (
         ctypes.c_int,
         [_PP, ctypes.POINTER(ctypes.c_int32), _PI64, _I32, _I32, _P, _I64, _P, _I32, _P],

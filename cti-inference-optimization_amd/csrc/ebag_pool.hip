@@ -1116,16 +1116,17 @@ __device__ __forceinline__ void wave_sync() { __builtin_amdgcn_wave_barrier(); }
 
 // WALK (rows of 64 lane vectors): a wavefront streams its bags' rows as the main kernel streams a tile
 // (stream_walk: uniform row addresses, K rows in flight across bags) instead of pooling them in rounds.
-template <typename TT, typename PT, int LANES, int SPW, bool BUF, bool WALK, int W = fused_waves(LANES)>
+// OT: the rows' type before and after the LayerNorm (the table's; bf16 for int8 tables, which are walked).
+template <typename TT, typename OT, typename PT, int LANES, int SPW, bool BUF, bool WALK, int W = fused_waves(LANES)>
 __global__ void __launch_bounds__(W * kWave) pool_norm_kernel(const PoolParams p, const FusedNorm fn) {
   using S = Shape<TT, LANES, 1>;
   constexpr int U = S::U;
   constexpr int R = S::R;
   static_assert(W >= 4, "a wavefront's list of short bags holds at most kFusedBags / 4 entries");
-  extern __shared__ uint4 s_row_raw[];  // the output rows: SPW * F * D elements of TT
+  extern __shared__ uint4 s_row_raw[];  // the output rows: SPW * F * D elements of OT
   __shared__ FusedLds s_w[W];
   __shared__ float s_red[W * SPW];
-  TT* const row = reinterpret_cast<TT*>(s_row_raw);
+  OT* const row = reinterpret_cast<OT*>(s_row_raw);
 
   const int wave = static_cast<int>(threadIdx.x) / kWave;
   const int lane = lane_id();
@@ -1178,7 +1179,7 @@ __global__ void __launch_bounds__(W * kWave) pool_norm_kernel(const PoolParams p
     const int n_mine = __popcll(__ballot(mine));
     const int bag = lane < n_mine ? s.order[lane] : 0;  // lane i: this wavefront's i-th bag
     const int64_t bs = shfl_i64(start, bag), be = shfl_i64(end, bag);
-    const WalkTable wt = walk_table(p.f[0], false, BUF);
+    const WalkTable wt = walk_table(p.f[0], Quantized<TT>::value, BUF);
     const auto write_bag = [&](int i, const float* r) {
       store_out<S::VEC>(row + static_cast<int64_t>(__builtin_amdgcn_readlane(bag, i)) * D + lane * S::VEC, r, false);
     };
@@ -1261,13 +1262,13 @@ __global__ void __launch_bounds__(W * kWave) pool_norm_kernel(const PoolParams p
   // LayerNorm of each row (online_best/infer.py:843-856): fp32 mean, fp32 variance of the
   // deviations, y = (x - mean) * rstd * gamma + beta rounded once to the output type. The rows
   // of the workgroup's samples share each gamma / beta load.
-  constexpr int VEC = 16 / Elem<TT>::kBytes;
+  constexpr int VEC = 16 / Elem<OT>::kBytes;
   const int cols = F * D;
   const int nvec = cols / VEC;
   const int t = static_cast<int>(threadIdx.x);
   constexpr int THREADS = W * kWave;
   const char* const rb = reinterpret_cast<const char*>(row);
-  const int64_t rstride = static_cast<int64_t>(cols) * Elem<TT>::kBytes;
+  const int64_t rstride = static_cast<int64_t>(cols) * Elem<OT>::kBytes;
   const float n = static_cast<float>(cols);
   // the SPW rows' sums share one workgroup reduction, then their squared deviations share one
   // (taking the sums while the rows are written held 4 more VGPRs: 7 wavefronts per SIMD)
@@ -1277,7 +1278,7 @@ __global__ void __launch_bounds__(W * kWave) pool_norm_kernel(const PoolParams p
     float sum = 0.f;
     for (int i = t; i < nvec; i += THREADS) {
       float x[VEC];
-      unpack16(load16(rb + j * rstride + i * 16), x, TT{});
+      unpack16(load16(rb + j * rstride + i * 16), x, OT{});
 #pragma unroll
       for (int e = 0; e < VEC; ++e) sum += x[e];
     }
@@ -1290,7 +1291,7 @@ __global__ void __launch_bounds__(W * kWave) pool_norm_kernel(const PoolParams p
     float q = 0.f;
     for (int i = t; i < nvec; i += THREADS) {
       float x[VEC];
-      unpack16(load16(rb + j * rstride + i * 16), x, TT{});
+      unpack16(load16(rb + j * rstride + i * 16), x, OT{});
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
         const float d = x[e] - mean[j];
@@ -1311,10 +1312,10 @@ __global__ void __launch_bounds__(W * kWave) pool_norm_kernel(const PoolParams p
       for (int j = 0; j < SPW; ++j) {
         if (b0 + j >= p.batch) break;
         float x[VEC], r[VEC];
-        unpack16(load16(rb + j * rstride + i * 16), x, TT{});
+        unpack16(load16(rb + j * rstride + i * 16), x, OT{});
 #pragma unroll
         for (int e = 0; e < VEC; ++e) r[e] = (x[e] - mean[j]) * rstd[j] * gm[e] + bt[e];
-        store_out<VEC>(reinterpret_cast<TT*>(p.out) + (b0 + j) * p.out_row_stride + static_cast<int64_t>(i) * VEC, r,
+        store_out<VEC>(reinterpret_cast<OT*>(p.out) + (b0 + j) * p.out_row_stride + static_cast<int64_t>(i) * VEC, r,
                        decltype(stream)::value);
       }
     }
@@ -2312,25 +2313,27 @@ int run_all_slots(const void* values, int32_t index_type, const void* val_offset
 namespace cti {
 namespace {
 
-template <typename TT, typename PT, int LANES>
+template <typename TT, typename OT, typename PT, int LANES>
 hipError_t launch_fused(const PoolParams& p, const FusedNorm& fn, int spw, size_t row_lds, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>((p.batch + spw - 1) / spw)), block(fused_waves(LANES) * kWave);
   const size_t lds = row_lds * spw;
   constexpr bool kWalk = LANES == kWave;
   if (kWalk && p.stream_ok) {
     switch (spw * 2 + (p.buffer_ok ? 1 : 0)) {
-      case 2: hipLaunchKernelGGL((pool_norm_kernel<TT, PT, LANES, 1, false, kWalk>), grid, block, lds, s, p, fn); break;
-      case 3: hipLaunchKernelGGL((pool_norm_kernel<TT, PT, LANES, 1, true, kWalk>), grid, block, lds, s, p, fn); break;
-      case 4: hipLaunchKernelGGL((pool_norm_kernel<TT, PT, LANES, 2, false, kWalk>), grid, block, lds, s, p, fn); break;
-      default: hipLaunchKernelGGL((pool_norm_kernel<TT, PT, LANES, 2, true, kWalk>), grid, block, lds, s, p, fn); break;
+      case 2: hipLaunchKernelGGL((pool_norm_kernel<TT, OT, PT, LANES, 1, false, kWalk>), grid, block, lds, s, p, fn); break;
+      case 3: hipLaunchKernelGGL((pool_norm_kernel<TT, OT, PT, LANES, 1, true, kWalk>), grid, block, lds, s, p, fn); break;
+      case 4: hipLaunchKernelGGL((pool_norm_kernel<TT, OT, PT, LANES, 2, false, kWalk>), grid, block, lds, s, p, fn); break;
+      default: hipLaunchKernelGGL((pool_norm_kernel<TT, OT, PT, LANES, 2, true, kWalk>), grid, block, lds, s, p, fn); break;
     }
     return hipGetLastError();
   }
-  switch (spw * 2 + (p.buffer_ok ? 1 : 0)) {
-    case 2: hipLaunchKernelGGL((pool_norm_kernel<TT, PT, LANES, 1, false, false>), grid, block, lds, s, p, fn); break;
-    case 3: hipLaunchKernelGGL((pool_norm_kernel<TT, PT, LANES, 1, true, false>), grid, block, lds, s, p, fn); break;
-    case 4: hipLaunchKernelGGL((pool_norm_kernel<TT, PT, LANES, 2, false, false>), grid, block, lds, s, p, fn); break;
-    default: hipLaunchKernelGGL((pool_norm_kernel<TT, PT, LANES, 2, true, false>), grid, block, lds, s, p, fn); break;
+  if constexpr (!Quantized<TT>::value) {
+    switch (spw * 2 + (p.buffer_ok ? 1 : 0)) {
+      case 2: hipLaunchKernelGGL((pool_norm_kernel<TT, OT, PT, LANES, 1, false, false>), grid, block, lds, s, p, fn); break;
+      case 3: hipLaunchKernelGGL((pool_norm_kernel<TT, OT, PT, LANES, 1, true, false>), grid, block, lds, s, p, fn); break;
+      case 4: hipLaunchKernelGGL((pool_norm_kernel<TT, OT, PT, LANES, 2, false, false>), grid, block, lds, s, p, fn); break;
+      default: hipLaunchKernelGGL((pool_norm_kernel<TT, OT, PT, LANES, 2, true, false>), grid, block, lds, s, p, fn); break;
+    }
   }
   return hipGetLastError();
 }
@@ -2339,11 +2342,11 @@ template <typename TT, typename PT>
 hipError_t launch_fused_lanes(int lanes, const PoolParams& p, const FusedNorm& fn, int spw, size_t row_lds,
                               hipStream_t s) {
   switch (lanes) {
-    case 4: return launch_fused<TT, PT, 4>(p, fn, spw, row_lds, s);
-    case 8: return launch_fused<TT, PT, 8>(p, fn, spw, row_lds, s);
-    case 16: return launch_fused<TT, PT, 16>(p, fn, spw, row_lds, s);
-    case 32: return launch_fused<TT, PT, 32>(p, fn, spw, row_lds, s);
-    default: return launch_fused<TT, PT, 64>(p, fn, spw, row_lds, s);
+    case 4: return launch_fused<TT, TT, PT, 4>(p, fn, spw, row_lds, s);
+    case 8: return launch_fused<TT, TT, PT, 8>(p, fn, spw, row_lds, s);
+    case 16: return launch_fused<TT, TT, PT, 16>(p, fn, spw, row_lds, s);
+    case 32: return launch_fused<TT, TT, PT, 32>(p, fn, spw, row_lds, s);
+    default: return launch_fused<TT, TT, PT, 64>(p, fn, spw, row_lds, s);
   }
 }
 
@@ -2365,13 +2368,16 @@ constexpr int kFusedMaxSlots = 64;
 }  // namespace
 }  // namespace cti
 
-extern "C" int cti_ebag_fused_all_slots_layernorm(const void* values, int32_t index_type, const void* val_offsets,
-                                                  const void* row_offsets, int32_t offset_type, const void* weight,
-                                                  int32_t dtype, void* out, int64_t batch_size, int32_t num_slots,
-                                                  int32_t emb_dim, int64_t max_idx, int64_t nnz, int32_t pooling,
-                                                  const void* gamma, const void* beta, int32_t param_dtype, float eps,
-                                                  void* stream) {
-  clear_error();
+namespace cti {
+namespace {
+
+// The fused pooling and LayerNorm launch; `dtype` is the rows' type before and after the LayerNorm,
+// `scale` the row scales of an int8 table (NULL: the table is of that type too).
+int run_fused_norm(const void* values, int32_t index_type, const void* val_offsets, const void* row_offsets,
+                   int32_t offset_type, const void* weight, const float* scale, int32_t dtype, void* out,
+                   int64_t batch_size, int32_t num_slots, int32_t emb_dim, int64_t max_idx, int64_t nnz,
+                   int32_t pooling, const void* gamma, const void* beta, int32_t param_dtype, float eps, void* stream,
+                   bool int8) {
   if (index_type != CTI_EBAG_I64 && index_type != CTI_EBAG_I32)
     return set_error(CTI_EBAG_EINVAL, "unknown index type code %d", index_type);
   if (offset_type != CTI_EBAG_I64 && offset_type != CTI_EBAG_I32)
@@ -2387,11 +2393,16 @@ extern "C" int cti_ebag_fused_all_slots_layernorm(const void* values, int32_t in
   if (nnz < 0) return set_error(CTI_EBAG_EINVAL, "nnz must be >= 0 (got %lld)", (long long)nnz);
   if (!(eps >= 0.0f)) return set_error(CTI_EBAG_EINVAL, "eps must be >= 0");
   if (batch_size == 0 || num_slots == 0) return CTI_EBAG_OK;
-  if (!val_offsets || !row_offsets || !weight || !out || !gamma || !beta || (nnz > 0 && !values))
-    return set_error(CTI_EBAG_EINVAL, "NULL device pointer among values/val_offsets/row_offsets/weight/out/gamma/beta");
+  if (!val_offsets || !row_offsets || !weight || !out || !gamma || !beta || (nnz > 0 && !values) ||
+      (int8 && !scale))
+    return set_error(CTI_EBAG_EINVAL, "NULL device pointer among values/val_offsets/row_offsets/weight/scale/out/gamma/beta");
   // shapes the fused kernel covers; the caller runs pooling and LayerNorm separately otherwise
   const int tb = dtype_bytes(dtype);
-  const int64_t row_bytes = static_cast<int64_t>(emb_dim) * tb;
+  const int64_t row_bytes = static_cast<int64_t>(emb_dim) * tb;  // of a pooled row
+  const int64_t table_row = int8 ? emb_dim : row_bytes;
+  if (int8 && (dtype != CTI_EBAG_BF16 || emb_dim != 8 * kWave || !stream_ids_ok(nnz, index_type == CTI_EBAG_I32)))
+    return set_error(CTI_EBAG_EUNSUPPORTED, "fused LayerNorm: int8 tables of other than %d columns, rows of another type than "
+                     "bf16, or a batch of 2^28 or more ids", 8 * kWave);
   if (dtype == CTI_EBAG_F16 || param_dtype == CTI_EBAG_F16)
     return set_error(CTI_EBAG_EUNSUPPORTED, "fused LayerNorm: fp16 tables or parameters");
   if (num_slots > kFusedMaxSlots)
@@ -2425,13 +2436,14 @@ extern "C" int cti_ebag_fused_all_slots_layernorm(const void* values, int32_t in
   p.block_threshold = kNoLimit;
   p.split_threshold = kNoLimit;
   const int64_t rows = max_idx + 1;
-  const int64_t span = (rows - 1) * row_bytes + row_bytes;
-  const bool fits = rows < (int64_t{1} << 32) / row_bytes;
+  const int64_t span = rows * table_row;
+  const bool fits = rows < (int64_t{1} << 32) / table_row;
   for (int f = 0; f < num_slots; ++f) {
     FieldDesc& d = p.f[f];
     d.table = static_cast<const char*>(weight);
     d.max_row = max_idx;
-    d.row_bytes = row_bytes;
+    d.row_scale = scale;
+    d.row_bytes = table_row;
     d.dim = emb_dim;
     d.out_col = f * emb_dim;
     d.gidx = f;
@@ -2447,7 +2459,10 @@ extern "C" int cti_ebag_fused_all_slots_layernorm(const void* values, int32_t in
   const int spw = fused_samples(num_slots, row_bytes * num_slots);
   hipStream_t st = static_cast<hipStream_t>(stream);
   hipError_t e;
-  if (dtype == CTI_EBAG_F32)
+  if (int8)
+    e = param_dtype == CTI_EBAG_F32 ? launch_fused<i8_t, bf16_t, float, kWave>(p, fn, spw, row_lds, st)
+                                    : launch_fused<i8_t, bf16_t, bf16_t, kWave>(p, fn, spw, row_lds, st);
+  else if (dtype == CTI_EBAG_F32)
     e = param_dtype == CTI_EBAG_F32 ? launch_fused_lanes<float, float>(lanes, p, fn, spw, row_lds, st)
                                     : launch_fused_lanes<float, bf16_t>(lanes, p, fn, spw, row_lds, st);
   else
@@ -2455,6 +2470,34 @@ extern "C" int cti_ebag_fused_all_slots_layernorm(const void* values, int32_t in
                                     : launch_fused_lanes<bf16_t, bf16_t>(lanes, p, fn, spw, row_lds, st);
   if (e != hipSuccess) return set_error(CTI_EBAG_EHIP, "fused pooling + LayerNorm launch failed: %s", hipGetErrorString(e));
   return CTI_EBAG_OK;
+}
+
+}  // namespace
+}  // namespace cti
+
+extern "C" int cti_ebag_fused_all_slots_layernorm(const void* values, int32_t index_type, const void* val_offsets,
+                                                  const void* row_offsets, int32_t offset_type, const void* weight,
+                                                  int32_t dtype, void* out, int64_t batch_size, int32_t num_slots,
+                                                  int32_t emb_dim, int64_t max_idx, int64_t nnz, int32_t pooling,
+                                                  const void* gamma, const void* beta, int32_t param_dtype, float eps,
+                                                  void* stream) {
+  clear_error();
+  return run_fused_norm(values, index_type, val_offsets, row_offsets, offset_type, weight, nullptr, dtype, out,
+                        batch_size, num_slots, emb_dim, max_idx, nnz, pooling, gamma, beta, param_dtype, eps, stream,
+                        false);
+}
+
+extern "C" int cti_ebag_fused_all_slots_layernorm_int8(const void* values, int32_t index_type, const void* val_offsets,
+                                                       const void* row_offsets, int32_t offset_type,
+                                                       const int8_t* weight_int8, const float* scale, void* out,
+                                                       int32_t out_dtype, int64_t batch_size, int32_t num_slots,
+                                                       int32_t emb_dim, int64_t max_idx, int64_t nnz, int32_t pooling,
+                                                       const void* gamma, const void* beta, int32_t param_dtype,
+                                                       float eps, void* stream) {
+  clear_error();
+  return run_fused_norm(values, index_type, val_offsets, row_offsets, offset_type, weight_int8, scale, out_dtype, out,
+                        batch_size, num_slots, emb_dim, max_idx, nnz, pooling, gamma, beta, param_dtype, eps, stream,
+                        true);
 }
 
 extern "C" int cti_ebag_fused_all_slots(const int64_t* values, const int64_t* val_offsets,

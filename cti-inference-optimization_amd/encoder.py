@@ -21,7 +21,8 @@ import torch
 from torch import nn
 
 from .layout import pack_slots
-from .ops import (fused_all_slots_embedding, fused_all_slots_embedding_int8, fused_all_slots_embedding_layernorm,
+from .ops import (fused_all_slots_embedding, fused_all_slots_embedding_int8,
+                  fused_all_slots_embedding_int8_layernorm, fused_all_slots_embedding_layernorm,
                   layer_norm, layer_norm_linear, layer_norm_stats, quantize_embedding_int8)
 
 
@@ -86,17 +87,18 @@ class RepEncoder(nn.Module):
         """Pooled rows after the input LayerNorm: ``[B, slot_num*emb_dim]`` in the table dtype.
 
         With the float table, pooling and LayerNorm run as one kernel (the pooled row stays on
-        chip); with the int8 table, the int8 pooling is followed by the LayerNorm kernel.
+        chip), as they do with an int8 table of 512 columns; with other int8 tables the int8 pooling
+        is followed by the LayerNorm kernel.
         """
         norm = self.input_norm
-        if self._int8_weight is not None:
-            fused_embs = self.pooled(batch)
-            with torch.no_grad():
-                return layer_norm(fused_embs, norm.weight.detach(), norm.bias.detach(), norm.eps, out=fused_embs)
         flat_values, val_offsets, flat_row_offsets, batch_size = self.flat_inputs(batch)
         weight = self.emb.weight
         out = torch.empty((batch_size, self.slot_num * self.emb_dim), device=weight.device, dtype=weight.dtype)
         with torch.no_grad():
+            if self._int8_weight is not None:
+                return fused_all_slots_embedding_int8_layernorm(
+                    flat_values, val_offsets, flat_row_offsets, self._int8_weight, self._int8_scale, out, batch_size,
+                    self.emb_dim, self.emb.num_embeddings - 1, norm.weight.detach(), norm.bias.detach(), norm.eps)
             return fused_all_slots_embedding_layernorm(flat_values, val_offsets, flat_row_offsets, weight.detach(), out,
                                                        batch_size, self.emb_dim, self.emb.num_embeddings - 1,
                                                        norm.weight.detach(), norm.bias.detach(), norm.eps)

@@ -394,6 +394,62 @@ def fused_all_slots_embedding_layernorm(
     return out
 
 
+def fused_all_slots_embedding_int8_layernorm(
+    flat_values: torch.Tensor,
+    val_offsets: torch.Tensor,
+    flat_row_offsets: torch.Tensor,
+    weight_int8: torch.Tensor,
+    scale: torch.Tensor,
+    out: torch.Tensor,
+    batch_size: int,
+    emb_dim: int,
+    max_idx: int,
+    ln_weight: torch.Tensor,
+    ln_bias: torch.Tensor,
+    eps: float = 1e-5,
+) -> torch.Tensor:
+    """``fused_all_slots_embedding_int8`` followed by the input LayerNorm (online_best/infer.py:904-942,
+    :1061-1076), sum pooling, into ``out`` [B, S*emb_dim].
+
+    Rows of 512 columns with a bf16 ``out`` run as one kernel, which keeps the pooled row on chip; other
+    shapes run the int8 pooling and the LayerNorm kernel one after the other, in place. Returns ``out``.
+    """
+    dev = weight_int8.device
+    num_slots = val_offsets.numel()
+    width = num_slots * emb_dim
+    if (emb_dim == 512 and out.dtype == torch.bfloat16 and tuple(out.shape) == (batch_size, width)
+            and ln_weight.dtype == ln_bias.dtype and ln_weight.dtype in (torch.bfloat16, torch.float32)):
+        _require_device_tensor("weight_int8", weight_int8)
+        icode, ocode = _check_flat_layout(flat_values, val_offsets, flat_row_offsets, out, dev)
+        val_offsets = _same_offset_type(val_offsets, flat_row_offsets, flat_values.numel())
+        for name, t in (("weight_int8", weight_int8), ("scale", scale), ("ln_weight", ln_weight), ("ln_bias", ln_bias)):
+            _require_device_tensor(name, t, dev)
+            _require_contiguous(name, t)
+        if weight_int8.dtype != torch.int8 or weight_int8.dim() != 2 or weight_int8.shape[1] != emb_dim:
+            raise TypeError(f"weight_int8 must be int8 [V, {emb_dim}] (got {weight_int8.dtype}, {tuple(weight_int8.shape)})")
+        if scale.dtype != torch.float32 or scale.numel() != weight_int8.shape[0]:
+            raise TypeError(f"scale must be float32 with {weight_int8.shape[0]} elements")
+        if not 0 <= max_idx < weight_int8.shape[0]:
+            raise ValueError(f"max_idx {max_idx} outside [0, {weight_int8.shape[0] - 1}]")
+        if flat_row_offsets.numel() != num_slots * (batch_size + 1):
+            raise ValueError(f"flat_row_offsets has {flat_row_offsets.numel()} entries, expected "
+                             f"{num_slots} * ({batch_size} + 1)")
+        if ln_weight.numel() != width or ln_bias.numel() != width:
+            raise ValueError(f"ln_weight / ln_bias must hold {width} elements")
+        with torch.cuda.device(dev):
+            rc = _capi.lib().cti_ebag_fused_all_slots_layernorm_int8(
+                flat_values.data_ptr(), icode, val_offsets.data_ptr(), flat_row_offsets.data_ptr(), ocode,
+                weight_int8.data_ptr(), scale.data_ptr(), out.data_ptr(), _capi.dtype_code(out.dtype), batch_size,
+                num_slots, emb_dim, max_idx, flat_values.numel(), _capi.SUM, ln_weight.data_ptr(), ln_bias.data_ptr(),
+                _capi.dtype_code(ln_weight.dtype), float(eps), _capi.current_stream_handle(dev))
+        if rc != _capi.EUNSUPPORTED:
+            _capi.check(rc)
+            return out
+    out = fused_all_slots_embedding_int8(flat_values, val_offsets, flat_row_offsets, weight_int8, scale, out, batch_size,
+                                         emb_dim, max_idx)
+    return layer_norm(out, ln_weight, ln_bias, eps, out=out)
+
+
 def fused_embedding(batch: dict, weight: torch.Tensor, slot_num: int, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """The fused embedding step of RepEncoder.forward (online_best/infer.py:1029-1059) on a
     batch dict holding ``_flat_values``, ``_flat_row_offsets`` and ``_val_offsets``.

@@ -350,6 +350,20 @@ int cti_ebag_fused_all_slots_layernorm(const void* values, int32_t index_type, c
                                        void* stream);
 
 /*
+ * cti_ebag_fused_all_slots_layernorm over an int8 table (rows as cti_ebag_fused_all_slots_int8 pools
+ * them: acc = fma(q, scale[row], acc) in element order, the sum rounded to bf16). Covered shapes: rows
+ * of 512 columns, bf16 output, gamma and beta of F32 or BF16, S <= 64, fewer than 2^28 ids (and 4 GiB
+ * of them), 16-byte aligned weight / out / gamma / beta; otherwise CTI_EBAG_EUNSUPPORTED (run
+ * cti_ebag_fused_all_slots_int8 and cti_ebag_layernorm instead).
+ */
+int cti_ebag_fused_all_slots_layernorm_int8(const void* values, int32_t index_type, const void* val_offsets,
+                                            const void* row_offsets, int32_t offset_type, const int8_t* weight_int8,
+                                            const float* scale, void* out, int32_t out_dtype, int64_t batch_size,
+                                            int32_t num_slots, int32_t emb_dim, int64_t max_idx, int64_t nnz,
+                                            int32_t pooling, const void* gamma, const void* beta, int32_t param_dtype,
+                                            float eps, void* stream);
+
+/*
  * Host-side compaction of sign ids for the transfer to the device (replaces the int64
  * `.to(device, non_blocking=True)` of `_flat_values` at online_best/infer.py:745-746; the comment
  * at :744 names the int32 form). `src` and `dst` are HOST pointers (dst typically pinned):

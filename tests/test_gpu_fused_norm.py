@@ -249,3 +249,36 @@ def test_wide_table_beyond_4_gib(pkg, dev, int8):
         out[name] = (enc.pooled(batch), enc.normalized(batch))
     for a, b in zip(out["big"], out["small"]):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+@pytest.mark.parametrize("B", [1, 9, 131])
+@pytest.mark.parametrize("S", [1, 5, 28, 64])
+@pytest.mark.parametrize("pdt", [torch.bfloat16, torch.float32])
+def test_fused_int8_layernorm_equals_two_launches(pkg, dev, B, S, pdt):
+    """Rows pooled and normalised in one launch: the pooled rows are the int8 pooling's (rounded to
+    bf16), so the result is the LayerNorm kernel's up to its fp32 rounding and one bf16 ulp."""
+    print(f"int8 fused norm B={B} S={S} params={pdt}", flush=True)
+    D, V = 512, 300
+    g = torch.Generator(device="cpu").manual_seed(B * 100 + S)
+    lens = torch.randint(0, 9, (S, B), generator=g)
+    lens[::3, ::5] = 70
+    rows = torch.zeros(S, B + 1, dtype=torch.int64)
+    rows[:, 1:] = torch.cumsum(lens, 1)
+    starts = (torch.cumsum(rows[:, -1], 0) - rows[:, -1]).to(dev)
+    ids = torch.randint(-2, V + 2, (int(lens.sum()),), generator=g).to(dev)
+    rows = rows.reshape(-1).to(dev)
+    q = torch.randint(-128, 128, (V, D), generator=g, dtype=torch.int8).to(dev)
+    scale = (torch.rand(V, generator=g) * 0.01 + 1e-4).to(dev)
+    gamma = (1 + 0.1 * torch.randn(S * D, generator=g)).to(dev).to(pdt)
+    beta = (0.1 * torch.randn(S * D, generator=g)).to(dev).to(pdt)
+    want = torch.empty(B, S * D, dtype=torch.bfloat16, device=dev)
+    pkg.fused_all_slots_embedding_int8(ids, starts, rows, q, scale, want, B, D, V - 1)
+    want = pkg.layer_norm(want, gamma, beta, 1e-5).double()
+    for idt in (torch.int64, torch.int32):
+        got = torch.full((B, S * D), float("nan"), dtype=torch.bfloat16, device=dev)
+        pkg.fused_all_slots_embedding_int8_layernorm(ids.to(idt), starts.to(idt), rows.to(idt), q, scale, got, B, D, V - 1,
+                                                     gamma, beta, 1e-5)
+        # the same pooled rows and formula, the sums in another order of fp32 additions (2e-5): values that
+        # close round to the same bf16 or to neighbours, which are at most 2^-7 of the larger apart
+        assert ((got.double() - want).abs() <= want.abs() * 2.0 ** -7 * (1 + 2.0 ** -7) + 2e-5).all()
+        assert (got.double() != want).double().mean() < 0.01
