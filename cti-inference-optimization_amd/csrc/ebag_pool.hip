@@ -567,7 +567,7 @@ __device__ __forceinline__ void store_lane(OT* dst, const float* a) {
 // is uniform, so its address costs no vector instruction; in rounds it cost every lane a 64-bit
 // product and the masking of each row (70 vector instructions a row in all, for 16 that unpack and
 // add). 28 slots of 512, 4,096 samples, mean length 8, pooled and normalised: 5 GB of bf16 143 -> 136 us
-// (5.2 TB/s of L2 misses), int8 148 -> 131 us.
+// (5.2 TB/s of L2 misses), int8 148 -> 131 us (121 as one launch with the LayerNorm).
 template <typename TT, int LANES, int VPL>
 struct StreamShape {
   static constexpr bool wide = LANES == 64 && VPL == 1;
@@ -2190,16 +2190,22 @@ int run_job(const Job& j, hipStream_t stream) {
       p.num_fields = static_cast<int32_t>(nf);
       p.wide_bags = p.stream_ok && !ordered ? kWideBags : bags_per_tile(kVarWide);
       bool all_buf = true;
-      int64_t tiles = 0;
+      int64_t tiles = 0, field_tiles = 0;
+      int last_bpt = 0;
       for (size_t i = 0; i < nf; ++i) {
         const int f = fields[c0 + i];
         const cti_ebag_table& t = j.tables[f];
         FieldDesc& d = p.f[i];
-        const int chunks = ragged_chunks(t.dim, tb == 1 ? 8 : 16 / tb);
+        const int chunks = v == kVarGeneric ? ragged_chunks(t.dim, tb == 1 ? 8 : 16 / tb) : 0;
         const int bpt = v == kVarGeneric ? ragged_side(chunks) : (v == kVarWide ? p.wide_bags : bags_per_tile(var[f]));
         d.lanes = v == kVarGeneric ? chunks : (var[f] <= 6 ? var[f] : 0);
         d.tile_begin = static_cast<int32_t>(tiles < INT32_MAX ? tiles : INT32_MAX);
-        tiles += v == kVarGeneric ? ((j.batch + bpt - 1) / bpt + 7) / 8 : (j.batch + bpt - 1) / bpt;
+        if (bpt != last_bpt) {  // one division per run of like fields
+          last_bpt = bpt;
+          field_tiles = (j.batch + bpt - 1) / bpt;
+          if (v == kVarGeneric) field_tiles = (field_tiles + 7) / 8;
+        }
+        tiles += field_tiles;
         d.table = static_cast<const char*>(t.data);
         d.row_scale = j.tdt == CTI_EBAG_I8 ? t.row_scale : nullptr;
         d.max_row = t.rows - 1;
@@ -2214,7 +2220,7 @@ int run_job(const Job& j, hipStream_t stream) {
         const bool fits = d.row_bytes >= 8 && t.rows < (int64_t{1} << 32) / d.row_bytes;
         // the ragged kernel's buffer loads: whole chunks of 4-byte aligned rows, and no offset from the
         // table's end on (span + a chunk's offset in the row) wraps around 32 bits
-        const bool ragged_buf = t.dim * tb >= 16 && reinterpret_cast<uintptr_t>(t.data) % 4 == 0 && d.row_bytes % 4 == 0 &&
+        const bool ragged_buf = v == kVarGeneric && t.dim * tb >= 16 && reinterpret_cast<uintptr_t>(t.data) % 4 == 0 && d.row_bytes % 4 == 0 &&
                                 span + static_cast<int64_t>(t.dim) * tb < (int64_t{1} << 32);
         d.span_bytes = (v == kVarGeneric ? ragged_buf : pow2 && fits) ? static_cast<uint32_t>(span) : 0u;
         all_buf = all_buf && d.span_bytes != 0;
