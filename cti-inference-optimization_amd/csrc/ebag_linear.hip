@@ -636,6 +636,7 @@ __global__ void __launch_bounds__(W * kWave, 2) ln_linear_band_kernel(const Line
   issue_w(0, first);
   issue_w(0, second);
   issue_x(1, ra[1]);
+  __builtin_amdgcn_sched_barrier(0);  // x of steps 2 and 3 is issued after all of these
   if constexpr (LN) {
     // gamma and beta of this workgroup's steps, 8 of each next to one another
     for (int i = t; i < nk * kChunks; i += THREADS) {
@@ -655,6 +656,10 @@ __global__ void __launch_bounds__(W * kWave, 2) ln_linear_band_kernel(const Line
   put_x(put_at + BM * kBK, ra[1], 0, PA);
   __builtin_amdgcn_sched_barrier(0);
   issue_x(3, ra[1]);
+  // The first half steps' waits count on the order of loads that the loop keeps; here the compiler orders
+  // them. So all but x of steps 2 and 3, the newest, have arrived before the loop, the weight in both
+  // halves among them (no longer a wait than that for x of step 1, which they were issued before).
+  wait_loads<2 * PA>();
   lds_barrier();
   constexpr int kAhead = 3;  // x fragments are read this many groups of products ahead
   // One half of step s: its fragments are read and the first products issued, which have then
