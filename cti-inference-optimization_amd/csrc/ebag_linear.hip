@@ -60,6 +60,7 @@ struct LinearParams {
   int32_t split_steps;  // split K: steps of kBK per split (even); split s is blockIdx.y
   int32_t bias_f32;     // bias is fp32 (else bf16)
   int32_t y_f32;        // y is fp32 (else bf16)
+  int32_t y_vec;        // y is aligned to 4 of its elements
 };
 
 // One bf16 chunk (8 elements) normalised: ((x - mean) * rstd) * g + b, rounded to bf16.
@@ -710,7 +711,9 @@ __global__ void __launch_bounds__(W * kWave, 2) ln_linear_band_kernel(const Line
 
   // lane l holds y[m0 + 16 a + l % 16][nw + 16 c + 4 (l / 16) + r]
   float* const part = p.part ? p.part + static_cast<int64_t>(blockIdx.y) * p.M * p.N : nullptr;
-  const bool whole = p.N % 4 == 0;  // then 4 columns starting at a multiple of 4 are all inside or all outside
+  // 4 columns starting at a multiple of 4 are all inside or all outside, and aligned (a caller's y need only
+  // be aligned to its elements; the partial products are)
+  const bool whole = p.N % 4 == 0 && (part || p.y_vec);
 #pragma unroll
   for (int c = 0; c < NI; ++c) {
     const int n = nw + c * 16 + fq * 4;
@@ -985,6 +988,7 @@ extern "C" int cti_ebag_layernorm_linear(const void* x, int64_t rows, int32_t co
   p.K = cols;
   p.bias_f32 = bias_dtype == CTI_EBAG_F32;
   p.y_f32 = y_dtype == CTI_EBAG_F32;
+  p.y_vec = reinterpret_cast<uintptr_t>(y) % (4 * (p.y_f32 ? 4 : 2)) == 0;
   p.part = workspace_bytes > 0 ? static_cast<float*>(workspace) : nullptr;
   hipStream_t s = static_cast<hipStream_t>(stream);
   hipError_t e;

@@ -246,3 +246,22 @@ def test_band_form_operands_exact(pkg, dev, rows, cols, n, pdt):
         for odt in (torch.float32, torch.bfloat16):
             got = pkg.layer_norm_linear(x, w, bias, out_dtype=odt, split_k=split_k, **kw)
             assert torch.equal(got, want.to(odt)), (split_k, odt)
+
+
+@pytest.mark.parametrize("rows,cols,n", [(24448, 128, 256), (16300, 128, 384), (16385, 128, 500), (2048, 7168, 384),
+                                         (300, 640, 512), (100, 200, 64)])
+@pytest.mark.parametrize("odt", [torch.float32, torch.bfloat16])
+def test_output_aligned_to_its_elements_alone(pkg, dev, rows, cols, n, odt):
+    """`out` from any element of a buffer on, in every form (the band form stores 4 elements at once where
+    it can): the result of an aligned `out`, and nothing written beside it."""
+    print(f"linear out offset rows={rows} cols={cols} n={n} out={odt}", flush=True)
+    g = torch.Generator(device="cpu").manual_seed(rows + n)
+    x = torch.randint(-3, 4, (rows, cols), generator=g, dtype=torch.int8).to(dev).to(torch.bfloat16)
+    w = torch.randint(-1, 2, (n, cols), generator=g, dtype=torch.int8).to(dev).to(torch.bfloat16)
+    want = (x.double() @ w.double().T).to(odt)
+    for split_k in (True, False):
+        for first in (1, 2, 3):
+            buf = torch.full((rows * n + 8,), float("nan"), dtype=odt, device=dev)
+            got = pkg.layer_norm_linear(x, w, out=buf[first:first + rows * n].view(rows, n), split_k=split_k)
+            assert torch.equal(got, want), (split_k, first)
+            assert buf[:first].isnan().all() and buf[first + rows * n:].isnan().all(), (split_k, first)
