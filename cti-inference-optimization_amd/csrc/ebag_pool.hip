@@ -73,6 +73,7 @@
 
 #include "ebag_device.h"
 #include "ebag_internal.h"
+#include "ebag_rules.h"
 
 namespace cti {
 namespace {
@@ -1710,7 +1711,7 @@ __device__ __forceinline__ void store_ragged(OT* dst, const float* r) {
   }
 }
 
-// BUF: rows at 4-byte aligned addresses of a float table of less than 4 GiB: byte offsets are staged
+// BUF: whole words at 4-byte aligned addresses (ragged_buffer_loads) of a float table: byte offsets are staged
 // in place of row ids and the rows read with buffer loads, past a bag's end at the table's end, which
 // reads zeros without a memory request.
 template <typename TT, typename OT, int C, bool BUF>
@@ -2218,10 +2219,8 @@ int run_job(const Job& j, hipStream_t stream) {
         // buffer path: power-of-two rows of >= 8 bytes and (rows + 1) * row_bytes <= 2^32, so the
         // pad row id 0xffffffff >> log2(row_bytes) addresses past both the rows and the scales
         const bool fits = d.row_bytes >= 8 && t.rows < (int64_t{1} << 32) / d.row_bytes;
-        // the ragged kernel's buffer loads: whole chunks of 4-byte aligned rows, and no offset from the
-        // table's end on (span + a chunk's offset in the row) wraps around 32 bits
-        const bool ragged_buf = v == kVarGeneric && t.dim * tb >= 16 && reinterpret_cast<uintptr_t>(t.data) % 4 == 0 && d.row_bytes % 4 == 0 &&
-                                span + static_cast<int64_t>(t.dim) * tb < (int64_t{1} << 32);
+        const bool ragged_buf = v == kVarGeneric && ragged_buffer_loads(reinterpret_cast<uintptr_t>(t.data), t.rows,
+                                                                        d.row_bytes, t.dim, tb);
         d.span_bytes = (v == kVarGeneric ? ragged_buf : pow2 && fits) ? static_cast<uint32_t>(span) : 0u;
         all_buf = all_buf && d.span_bytes != 0;
       }
