@@ -60,7 +60,6 @@ struct LinearParams {
   int32_t split_steps;  // split K: steps of kBK per split (even); split s is blockIdx.y
   int32_t bias_f32;     // bias is fp32 (else bf16)
   int32_t y_f32;        // y is fp32 (else bf16)
-  int32_t y_vec;        // y is aligned to 4 of its elements
 };
 
 // One bf16 chunk (8 elements) normalised: ((x - mean) * rstd) * g + b, rounded to bf16.
@@ -486,6 +485,10 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Vectors at any element's alignment: rows of y start at any multiple of its elements.
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
+typedef u32x2 u32x2_any __attribute__((aligned(2)));
+
 constexpr int kBandParams = 28 * 1024;  // LDS for gamma and beta (160 KB in all)
 
 // Waits until at most N of this wavefront's loads are in flight: all but the N newest have arrived, those to
@@ -711,9 +714,6 @@ __global__ void __launch_bounds__(W * kWave, 2) ln_linear_band_kernel(const Line
 
   // lane l holds y[m0 + 16 a + l % 16][nw + 16 c + 4 (l / 16) + r]
   float* const part = p.part ? p.part + static_cast<int64_t>(blockIdx.y) * p.M * p.N : nullptr;
-  // 4 columns starting at a multiple of 4 are all inside or all outside, and aligned (a caller's y need only
-  // be aligned to its elements; the partial products are)
-  const bool whole = p.N % 4 == 0 && (part || p.y_vec);
 #pragma unroll
   for (int c = 0; c < NI; ++c) {
     const int n = nw + c * 16 + fq * 4;
@@ -735,19 +735,20 @@ __global__ void __launch_bounds__(W * kWave, 2) ln_linear_band_kernel(const Line
       f32x4 v = acc[a][c];
 #pragma unroll
       for (int r = 0; r < 4; ++r) v[r] += bias[r];
+      const bool whole = n + 4 <= p.N;  // else the row's last 1 to 3 columns
       if (part || p.y_f32) {
         float* const y = (part ? part : reinterpret_cast<float*>(p.y)) + at;
         if (whole) {
-          *reinterpret_cast<f32x4*>(y) = v;
+          *reinterpret_cast<f32x4_any*>(y) = v;
         } else {
-          for (int r = 0; r < 4 && n + r < p.N; ++r) y[r] = v[r];
+          for (int r = 0; r < 3 && n + r < p.N; ++r) y[r] = v[r];
         }
       } else {
         uint16_t* const y = reinterpret_cast<uint16_t*>(p.y) + at;
         if (whole) {
-          *reinterpret_cast<u32x2*>(y) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+          *reinterpret_cast<u32x2_any*>(y) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
         } else {
-          for (int r = 0; r < 4 && n + r < p.N; ++r) y[r] = static_cast<uint16_t>(pack_bf16x2(v[r], 0.f));
+          for (int r = 0; r < 3 && n + r < p.N; ++r) y[r] = static_cast<uint16_t>(pack_bf16x2(v[r], 0.f));
         }
       }
     }
@@ -988,7 +989,6 @@ extern "C" int cti_ebag_layernorm_linear(const void* x, int64_t rows, int32_t co
   p.K = cols;
   p.bias_f32 = bias_dtype == CTI_EBAG_F32;
   p.y_f32 = y_dtype == CTI_EBAG_F32;
-  p.y_vec = reinterpret_cast<uintptr_t>(y) % (4 * (p.y_f32 ? 4 : 2)) == 0;
   p.part = workspace_bytes > 0 ? static_cast<float*>(workspace) : nullptr;
   hipStream_t s = static_cast<hipStream_t>(stream);
   hipError_t e;
