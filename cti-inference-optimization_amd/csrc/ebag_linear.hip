@@ -11,23 +11,24 @@
 // output). Without statistics the kernel is the plain Linear.
 //
 // Three forms (the products on v_mfma_f32_16x16x32_bf16: lane l supplies A[l%16][8(l/16) .. +8)
-// and B[8(l/16) .. +8)[l%16] and receives C[4(l/16) + r][l%16], r < 4; workgroups numbered so
-// that the tiles of one row band run on one XCD, whose L2 then serves the band to each of them):
-//   ln_linear_band_kernel many rows, K a multiple of 128: bands of 128 rows by 256, 384 or 512
-//                         columns, the weight loaded straight to LDS;
-//   ln_linear_big_kernel  K a multiple of 128, fewer rows: 128 x 256 or 128 x 128 tiles of 8
-//                         wavefronts, both operands through LDS (XOR-swizzled rows);
+// and B[8(l/16) .. +8)[l%16] and receives C[4(l/16) + r][l%16], r < 4), chosen by linear_plan:
+//   ln_linear_band_kernel K a multiple of 128: bands of 128 rows by 256, 384 or 512 columns, the
+//                         weight loaded straight to LDS;
+//   ln_linear_big_kernel  K a multiple of 128: 128 x 256 or 128 x 128 tiles of 8 wavefronts, both
+//                         operands through LDS (XOR-swizzled rows);
 //   ln_linear_kernel      any K (a multiple of 8): 64 x 256 tiles of 4 wavefronts, each owning 64
 //                         columns, x through LDS and the weight's fragments straight to registers.
 // The last two walk K in steps of 64 with each step's loads issued two steps ahead into rotating
-// register sets, x normalised on its way to LDS, two LDS buffers and one barrier per step. When the
-// tiles would leave CUs idle (few rows), K is split over several workgroups per tile: each
-// writes its fp32 partial products to a caller's workspace and ln_linear_reduce_kernel adds the
-// splits in split order, adds the bias and rounds once.
+// register sets, x normalised on its way to LDS, two LDS buffers and one barrier per step, and
+// number their workgroups so that the tiles of one row band run on one XCD, whose L2 then serves the
+// band to each of them. When the tiles would leave CUs idle (few rows), K is split over several
+// workgroups per tile: each writes its fp32 partial products to a caller's workspace and
+// ln_linear_reduce_kernel adds the splits in split order, adds the bias and rounds once.
 #include <stdint.h>
 
 #include "ebag_device.h"
 #include "ebag_internal.h"
+#include "ebag_rules.h"
 
 namespace cti {
 namespace {
@@ -35,12 +36,11 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kBK = 64;        // K per step
+constexpr int kBK = kLinearStep;  // K per step
 constexpr int kLds = kBK + 8;  // LDS row pitch in elements (144 bytes)
 constexpr int kChunks = kBK / 8;  // 16-byte chunks per tile row
 constexpr int kXcds = 8;
 constexpr int kWaveCols = 64;  // output columns per wavefront
-constexpr int64_t kSplitTarget = 256;  // split K until the large form has one workgroup per CU
 
 struct LinearParams {
   const char* x;      // [M, K] bf16
@@ -489,7 +489,7 @@ __device__ __forceinline__ void lds_barrier() {
 typedef f32x4 f32x4_any __attribute__((aligned(4)));
 typedef u32x2 u32x2_any __attribute__((aligned(2)));
 
-constexpr int kBandParams = 28 * 1024;  // LDS for gamma and beta (160 KB in all)
+constexpr int kBandParams = kLinearBandParams;  // LDS for gamma and beta (160 KB in all)
 
 // Waits until at most N of this wavefront's loads are in flight: all but the N newest have arrived, those to
 // LDS included (the compiler does not follow every load to LDS around a loop).
@@ -834,88 +834,22 @@ hipError_t launch_tile(LinearParams p, hipStream_t s) {
   return hipGetLastError();
 }
 
-// The large form applies to K a multiple of 128 with byte offsets below 2^31 (every encoder shape:
-// K = 28 * D).
-bool big_form(int64_t M, int32_t N, int32_t K) {
-  return K % (2 * kBK) == 0 && (M + 128) * K * 2 < (int64_t{1} << 31) && static_cast<int64_t>(N) * K * 2 < (int64_t{1} << 31);
-}
-
-// Column fragments per wavefront of the band form: 8 wavefronts cover N = 256, 384 or 512 columns.
-int band_fragments(int32_t N) { return N <= 256 ? 2 : (N <= 384 ? 3 : 4); }
-
-int64_t band_tiles(int64_t M, int32_t N) {
-  const int bn = 128 * band_fragments(N);
-  return (M + 127) / 128 * ((N + bn - 1) / bn);
-}
-
-// Split K into at most `want` parts of even step counts, as many as `ws_bytes` of fp32 partials hold;
-// 1 = no split. `steps` receives the steps per split.
-int split_count(int64_t want, int64_t M, int32_t N, int32_t K, int64_t ws_bytes, int* steps) {
-  const int nk = K / kBK;
-  *steps = nk;
-  if (want <= 1 || nk < 4) return 1;
-  const int64_t fit = ws_bytes / (M * N * 4);
-  if (want > fit) want = fit;
-  if (want > nk / 2) want = nk / 2;
-  if (want <= 1) return 1;
-  const int per = static_cast<int>(((nk + want - 1) / want + 1) / 2 * 2);  // even steps per split
-  *steps = per;
-  return (nk + per - 1) / per;
-}
-
-// The band form where it is the fastest: from about a workgroup per CU on (its 128 x 512 tiles; narrower
-// ones from 192 tiles), and below that, with K split, where tiles times steps of K outweigh the partial
-// products (N = 384, three of the other form's 128-column tiles: a quarter of that). Measured, bf16
-// parameters, us of the 128 x 128 / 128 x 256 form against this one:
-//   K = 3584, M = 30000   N = 256 / 384 / 512: 104 / 151 / 200 against 66 / 90 / 112
-//   K = 896, M = 30000    N = 256 / 384 / 512: 34 / 50 / 64 against 24 / 33 / 42
-//   M = 16384, N = 512    K = 896 / 1792 / 3584: 33 / 55 / 101 against 33 / 51 / 84 (2 splits)
-//   M = 8192              N = 384, K = 3584: 62 against 45; N = 512, K = 7168: 96 against 82;
-//                         N = 512, K = 3584: 51 against 58 (kept with the 128 x 128 tiles)
-bool band_form(int64_t M, int32_t N, int32_t K, int param_bytes) {
-  if (!big_form(M, N, K) || static_cast<int64_t>(K) * 2 * param_bytes > kBandParams) return false;
-  const int ni = band_fragments(N);
-  const int64_t tiles = band_tiles(M, N);
-  return tiles >= (ni == 2 ? 192 : 128) || tiles * (K / kBK) >= (ni == 3 ? 1792 : 7168);
-}
-
-// The band form's K splits: as many as keep its workgroups within one per CU.
-int band_splits(int64_t M, int32_t N, int32_t K, int64_t ws_bytes, int* steps) {
-  return split_count(kSplitTarget / band_tiles(M, N), M, N, K, ws_bytes, steps);
-}
-
-// The 128 x 128 tiles' K splits: enough for one workgroup per CU. (Two per CU measured slower: M = 1024,
-// K = 3584, N = 512 took 28.0 against 18.7 us, the partials' HBM traffic outweighing the extra
-// parallelism.)
-int tile_splits(int64_t M, int32_t N, int32_t K, int64_t ws_bytes, int* steps) {
-  const int64_t tiles = (M + 127) / 128 * ((N + 127) / 128);
-  return split_count((kSplitTarget + tiles - 1) / tiles, M, N, K, ws_bytes, steps);
-}
-
-// 128 x 256 tiles when there are at least two per CU, else 128 x 128 (split over K when even
-// those leave CUs idle), where the band form does not apply; the general form for the rest.
+// The form and the splits that linear_plan chooses for the shape and the workspace.
 template <bool LN, typename PT, typename BT, typename OT>
-hipError_t launch_linear(const LinearParams& p, int64_t ws_bytes, hipStream_t s) {
-  if (band_form(p.M, p.N, p.K, LN ? Elem<PT>::kBytes : 0)) {
-    LinearParams q = p;
-    int steps = 0;
-    const int splits = p.part ? band_splits(p.M, p.N, p.K, ws_bytes, &steps) : 1;
-    q.split_steps = steps;
-    switch (band_fragments(p.N)) {
-      case 2: return launch_band<2, LN, PT, BT, OT>(q, splits, s);
-      case 3: return launch_band<3, LN, PT, BT, OT>(q, splits, s);
-      default: return launch_band<4, LN, PT, BT, OT>(q, splits, s);
-    }
+hipError_t launch_linear(LinearParams p, int64_t ws_bytes, hipStream_t s) {
+  const LinearPlan plan = linear_plan(p.M, p.N, p.K, LN ? Elem<PT>::kBytes : 0, p.part ? ws_bytes : 0);
+  p.split_steps = plan.steps;
+  switch (plan.form) {
+    case kLinearBand:
+      switch (linear_band_fragments(p.N)) {
+        case 2: return launch_band<2, LN, PT, BT, OT>(p, plan.splits, s);
+        case 3: return launch_band<3, LN, PT, BT, OT>(p, plan.splits, s);
+        default: return launch_band<4, LN, PT, BT, OT>(p, plan.splits, s);
+      }
+    case kLinearTile256: return launch_big<256, 4, 2, LN, PT, BT, OT>(p, 1, s);
+    case kLinearTile128: return launch_big<128, 4, 2, LN, PT, BT, OT>(p, plan.splits, s);
+    default: return launch_tile<64, 4, 2, LN, PT, BT, OT>(p, s);
   }
-  if (big_form(p.M, p.N, p.K)) {
-    if ((p.M + 127) / 128 * ((p.N + 255) / 256) >= 2 * 256) return launch_big<256, 4, 2, LN, PT, BT, OT>(p, 1, s);
-    LinearParams q = p;
-    int steps = 0;
-    const int splits = p.part ? tile_splits(p.M, p.N, p.K, ws_bytes, &steps) : 1;
-    q.split_steps = steps;
-    return launch_big<128, 4, 2, LN, PT, BT, OT>(q, splits, s);
-  }
-  return launch_tile<64, 4, 2, LN, PT, BT, OT>(p, s);
 }
 
 template <bool LN, typename PT, typename BT>
@@ -934,15 +868,8 @@ hipError_t launch_bias(int32_t bdt, int32_t odt, const LinearParams& p, int64_t 
 using namespace cti;
 
 extern "C" int64_t cti_ebag_layernorm_linear_workspace_bytes(int64_t rows, int32_t cols, int32_t out_features) {
-  if (rows < 1 || cols < 1 || out_features < 1 || !big_form(rows, out_features, cols)) return 0;
-  int steps = 0;
-  // for whichever form the type of gamma and beta then selects
-  int splits = tile_splits(rows, out_features, cols, INT64_MAX, &steps);
-  if (band_form(rows, out_features, cols, 0)) {
-    const int band = band_splits(rows, out_features, cols, INT64_MAX, &steps);
-    if (band > splits || band_form(rows, out_features, cols, 4)) splits = band;
-  }
-  return splits > 1 ? static_cast<int64_t>(splits) * rows * out_features * 4 : 0;
+  if (rows < 1 || cols < 1 || out_features < 1) return 0;
+  return linear_workspace_bytes(rows, out_features, cols);
 }
 
 extern "C" int cti_ebag_layernorm_linear(const void* x, int64_t rows, int32_t cols, const float* mean,

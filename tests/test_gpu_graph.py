@@ -105,11 +105,13 @@ def test_reference_layout_and_fused_layernorm_replay(pkg, dev):
             assert torch.equal(normed.view(torch.int16), want_n.view(torch.int16)), rep
 
 
-@pytest.mark.parametrize("rows,cols,n", [(96, 3584, 512), (4096, 3584, 512), (300, 136, 64)])
+@pytest.mark.parametrize("rows,cols,n", [(96, 3584, 512), (4096, 3584, 512), (300, 136, 64), (8192, 7168, 512),
+                                         (16384, 1792, 512)])
 def test_layernorm_linear_replays(pkg, dev, rows, cols, n):
     """Statistics pass + LayerNorm-Linear captured together: K split over workgroups (workspace from
     the graph's pool, a GEMM and a reduction launch per call; 96 and 4096 rows), one launch
-    without a split (the general form, K not a multiple of 128). Every replay on new inputs
+    without a split (the general form, K not a multiple of 128), and the band form with K split (8192
+    rows) and whole (16384). Every replay on new inputs
     equals the eager call bit for bit."""
     print(f"layernorm-linear replay rows={rows} cols={cols} n={n}", flush=True)
     gen = torch.Generator().manual_seed(rows + cols)

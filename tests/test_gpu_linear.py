@@ -216,9 +216,9 @@ def test_split_k_uses_as_many_splits_as_the_workspace_holds(pkg, dev):
         assert torch.equal(y, want), ws_bytes
 
 
-# the band form's edges: its three column widths, tile counts beside the rule's limits, rows and columns
-# that are no whole tiles (also no multiple of 4), two column tiles, the smallest K, K split (rows from
-# 2,048 on), and parameters too large for its LDS copy
+# the band form's edges: its three column widths, rows and columns that are no whole tiles (also no
+# multiple of 4), two column tiles, the smallest K, K split, and parameters too large for its LDS copy (some
+# of these take the tiles, as test_dispatch_rules.py lists: the edges of the choice are here as well)
 BAND_SHAPES = [(24449, 128, 256), (24448, 256, 130), (16257, 128, 384), (16256, 384, 290), (16300, 640, 511),
                (16385, 128, 500), (8200, 256, 700), (2048, 7168, 384), (8192, 7168, 512), (16384, 3584, 512)]
 
@@ -246,6 +246,88 @@ def test_band_form_operands_exact(pkg, dev, rows, cols, n, pdt):
         for odt in (torch.float32, torch.bfloat16):
             got = pkg.layer_norm_linear(x, w, bias, out_dtype=odt, split_k=split_k, **kw)
             assert torch.equal(got, want.to(odt)), (split_k, odt)
+
+
+# shapes of the band form, K whole and split, with bf16 / fp32 / no LayerNorm (test_dispatch_rules.py holds
+# the library's choice to this list)
+BAND_WHOLE = [(30001, 128, 384, (2, 4, 0)), (30000, 384, 129, (2, 4)), (26000, 640, 511, (2, 4)),
+              (16390, 3584, 512, (2, 4)), (40000, 256, 1000, (2, 4, 0))]
+BAND_SPLIT = [(2047, 7168, 384, (2,)), (8192, 7168, 512, (2,)), (4100, 3584, 300, (2, 4)), (7000, 3584, 650, (2, 4))]
+_PARAM_DT = {2: torch.bfloat16, 4: torch.float32}
+
+
+def _band_cases(shapes):
+    return [(rows, cols, n, size) for rows, cols, n, sizes in shapes for size in sizes]
+
+
+@pytest.mark.parametrize("rows,cols,n,size", _band_cases(BAND_WHOLE + BAND_SPLIT))
+def test_band_form_realistic_operands(pkg, dev, rows, cols, n, size):
+    """Real-valued operands against float64 on the GPU, with the kernel's own statistics: the normalised
+    operand is the LayerNorm kernel's bit for bit, so the result meets the fp32 accumulation bound (as in
+    test_realistic_operands_against_the_oracle), whole and split, and repeats bit for bit."""
+    print(f"band realistic rows={rows} cols={cols} n={n} params={size}", flush=True)
+    x, gamma, beta, w, bias = _realistic(rows, cols, n, rows + n, dev)
+    kw, a = {}, x
+    if size:
+        gamma, beta = gamma.to(_PARAM_DT[size]), beta.to(_PARAM_DT[size])
+        mean, rstd = pkg.layer_norm_stats(x, 1e-5)
+        kw = dict(mean=mean, rstd=rstd, norm_weight=gamma, norm_bias=beta)
+        a = pkg.layer_norm(x, gamma, beta, 1e-5)
+    ref = a.double() @ w.double().T + bias.double()
+    # K products and the bias, each addition within 2^-23 of its partial sum; one more per split
+    bound = (cols + 64) * 2.0 ** -23 * (a.double().abs() @ w.double().abs().T + bias.double().abs())
+    for split_k in (True, False):
+        y32 = pkg.layer_norm_linear(x, w, bias, out_dtype=torch.float32, split_k=split_k, **kw)
+        y16 = pkg.layer_norm_linear(x, w, bias, split_k=split_k, **kw)
+        assert bool(((y32.double() - ref).abs() <= bound).all()), split_k
+        assert torch.equal(y16, y32.to(torch.bfloat16)), split_k  # one rounding of the same sums
+        again = pkg.layer_norm_linear(x, w, bias, split_k=split_k, **kw)
+        assert torch.equal(y16.view(torch.int16), again.view(torch.int16)), split_k
+
+
+def test_band_form_operands_exact_without_layer_norm(pkg, dev):
+    """Integer operands in the plain band form's three widths, odd columns among them."""
+    for rows, cols, n, sizes in BAND_WHOLE:
+        if 0 not in sizes:
+            continue
+        print(f"band exact plain rows={rows} cols={cols} n={n}", flush=True)
+        g = torch.Generator(device="cpu").manual_seed(rows + n)
+        x = torch.randint(-3, 4, (rows, cols), generator=g, dtype=torch.int8).to(dev).to(torch.bfloat16)
+        w = torch.randint(-1, 2, (n, cols), generator=g, dtype=torch.int8).to(dev).to(torch.bfloat16)
+        want = x.double() @ w.double().T
+        for odt in (torch.float32, torch.bfloat16):
+            assert torch.equal(pkg.layer_norm_linear(x, w, out_dtype=odt), want.to(odt)), odt
+
+
+@pytest.mark.parametrize("rows,cols,n,size", _band_cases(BAND_SPLIT))
+def test_band_form_workspaces_smaller_than_queried(pkg, dev, rows, cols, n, size):
+    """Any workspace: fewer splits, another form or none, the same result on integer operands."""
+    print(f"band workspaces rows={rows} cols={cols} n={n} params={size}", flush=True)
+    c = pkg._capi
+    full = c.lib().cti_ebag_layernorm_linear_workspace_bytes(rows, cols, n)
+    one = rows * n * 4
+    assert full >= 2 * one
+    g = torch.Generator(device="cpu").manual_seed(rows)
+    x = torch.randint(-3, 4, (rows, cols), generator=g, dtype=torch.int8).to(dev).to(torch.bfloat16)
+    w = torch.randint(-1, 2, (n, cols), generator=g, dtype=torch.int8).to(dev).to(torch.bfloat16)
+    mean = torch.randint(-2, 3, (rows,), generator=g).float().to(dev)
+    rstd = (1 + torch.randint(0, 2, (rows,), generator=g)).float().to(dev)
+    gamma = torch.randint(1, 3, (cols,), generator=g).to(dev).to(_PARAM_DT[size])
+    beta = torch.randint(-4, 5, (cols,), generator=g).to(dev).to(_PARAM_DT[size])
+    a = (x.double() - mean[:, None]) * rstd[:, None] * gamma.double() + beta.double()
+    want = (a @ w.double().T).float()
+    stream = c.current_stream_handle(dev)
+    for ws_bytes in (full, full - 16, 3 * one, 2 * one + 4096, 2 * one, one, 16):
+        print(f"workspace {ws_bytes} bytes", flush=True)
+        ws = torch.empty(ws_bytes + 64, dtype=torch.uint8, device=dev)
+        ws[ws_bytes:] = 123
+        y = torch.full((rows, n), float("nan"), dtype=torch.float32, device=dev)
+        c.check(c.lib().cti_ebag_layernorm_linear(
+            x.data_ptr(), rows, cols, mean.data_ptr(), rstd.data_ptr(), gamma.data_ptr(), beta.data_ptr(),
+            c.dtype_code(gamma.dtype), w.data_ptr(), n, None, c.F32, y.data_ptr(), c.F32, ws.data_ptr(), ws_bytes,
+            stream))
+        assert torch.equal(y, want), ws_bytes
+        assert bool((ws[ws_bytes:] == 123).all()), ws_bytes
 
 
 @pytest.mark.parametrize("rows,cols,n", [(24448, 128, 256), (16300, 128, 384), (16385, 128, 500), (2048, 7168, 384),
