@@ -2104,21 +2104,17 @@ int run_job(const Job& j, hipStream_t stream) {
   // Group fields by kernel variant; each group is one launch sequence (per 64 fields). Fields
   // whose rows are one lane vector per lane but of different widths form one mixed group.
   std::vector<int> var(j.num_fields);
-  for (int f = 0; f < j.num_fields; ++f) var[f] = pick_variant(j.tables[f], tb, ob, j.out, j.out_row_stride);
+  unsigned present = 0;  // bit v: a field of variant v
+  for (int f = 0; f < j.num_fields; ++f) {
+    var[f] = pick_variant(j.tables[f], tb, ob, j.out, j.out_row_stride);
+    present |= 1u << var[f];
+  }
   // Fields of the streamed shape that may take streamed tiles keep a launch of their own, so a field is
   // pooled the same way whatever other fields share the call.
   const bool stream_apart = stream_variant_allowed(j);
-  int one_vec_shapes = 0;
-  for (int v = kMixedLo; v <= kMixedHi; ++v) {
-    if (stream_apart && v == kVarStream) continue;
-    for (int f = 0; f < j.num_fields; ++f) {
-      if (var[f] == v) {
-        ++one_vec_shapes;
-        break;
-      }
-    }
-  }
-  const bool mixed = one_vec_shapes > 1;
+  unsigned mixable = (2u << kMixedHi) - (1u << kMixedLo);
+  if (stream_apart) mixable &= ~(1u << kVarStream);
+  const bool mixed = __builtin_popcount(present & mixable) > 1;
   // A dispatch order belongs to a job that is one main-kernel launch of one fixed row shape.
   const bool ordered = j.tile_order || j.next_order;
   if (ordered) {
@@ -2136,19 +2132,22 @@ int run_job(const Job& j, hipStream_t stream) {
       return set_error(CTI_EBAG_EINVAL, "order buffers of %lld bytes; this job needs %lld", (long long)j.order_bytes,
                        (long long)((kOrderHeader + tiles) * 4));
   }
+  std::vector<int> fields;
+  fields.reserve(j.num_fields);
   for (int v = 0; v <= kVarMixed; ++v) {
-    std::vector<int> fields;
+    fields.clear();
+    const bool ragged = v == kVarGeneric;
     if (v == kVarMixed) {
       if (!mixed) continue;
       // widest rows first (fewest bags per tile), so those tiles start first
       for (int w = kMixedHi; w >= kMixedLo; --w) {
-        if (stream_apart && w == kVarStream) continue;
+        if (!(present & mixable & 1u << w)) continue;
         for (int f = 0; f < j.num_fields; ++f) if (var[f] == w) fields.push_back(f);
       }
     } else {
-      if (mixed && v >= kMixedLo && v <= kMixedHi && !(stream_apart && v == kVarStream)) continue;
+      if (!(present & 1u << v) || (mixed && (mixable & 1u << v))) continue;
       for (int f = 0; f < j.num_fields; ++f) if (var[f] == v) fields.push_back(f);
-      if (v == kVarGeneric)  // narrowest rows first (see pool_ragged_kernel)
+      if (ragged)  // narrowest rows first (see pool_ragged_kernel)
         std::stable_sort(fields.begin(), fields.end(), [&](int a, int b) { return j.tables[a].dim < j.tables[b].dim; });
     }
     for (size_t c0 = 0; c0 < fields.size(); c0 += kMaxFields) {
@@ -2166,18 +2165,18 @@ int run_job(const Job& j, hipStream_t stream) {
       p.idx32 = j.idx32;
       p.off32 = j.off32;
       p.round_bf16 = j.round_bf16;
-      const bool bins = j.use_bins && v != kVarGeneric;
+      const bool bins = j.use_bins && !ragged;
       p.stream_ok = stream_variant_allowed(j) ? 1 : 0;
       p.stream_out = j.batch * j.out_row_stride * dtype_bytes(j.odt) >= kStreamOutBytes;
-      if (v == kVarGeneric) p.sub_threshold = kNoLimit;
+      if (ragged) p.sub_threshold = kNoLimit;
       else if (j.sub_threshold == 0) p.sub_threshold = default_sub_threshold(v, bins);
       else p.sub_threshold = j.sub_threshold < 0 ? 0 : j.sub_threshold;
       p.block_threshold = !bins ? kNoLimit : (j.block_threshold > 0 ? j.block_threshold : kDefaultBlockThreshold);
       p.split_threshold = !bins ? kNoLimit : (j.split_threshold > 0 ? j.split_threshold : kDefaultSplitThreshold);
       // a bag is pooled by exactly one kernel: never call a listed (long) bag short
-      if (v != kVarGeneric && p.sub_threshold > p.block_threshold) p.sub_threshold = p.block_threshold;
+      if (!ragged && p.sub_threshold > p.block_threshold) p.sub_threshold = p.block_threshold;
       // short-bag lengths are kept in 32 bits on the device
-      if (v != kVarGeneric && p.sub_threshold > kMaxShortBag) p.sub_threshold = kMaxShortBag;
+      if (!ragged && p.sub_threshold > kMaxShortBag) p.sub_threshold = kMaxShortBag;
       p.bin_count = bins ? list.count : nullptr;
       p.bin_total = bins ? list.total : nullptr;
       if (ordered) {  // the job's only launch: fields 0 .. F-1 in job order
@@ -2197,14 +2196,13 @@ int run_job(const Job& j, hipStream_t stream) {
         const int f = fields[c0 + i];
         const cti_ebag_table& t = j.tables[f];
         FieldDesc& d = p.f[i];
-        const int chunks = v == kVarGeneric ? ragged_chunks(t.dim, tb == 1 ? 8 : 16 / tb) : 0;
-        const int bpt = v == kVarGeneric ? ragged_side(chunks) : (v == kVarWide ? p.wide_bags : bags_per_tile(var[f]));
-        d.lanes = v == kVarGeneric ? chunks : (var[f] <= 6 ? var[f] : 0);
+        d.lanes = ragged ? ragged_chunks(t.dim, tb == 1 ? 8 : 16 / tb) : (var[f] <= 6 ? var[f] : 0);
+        const int bpt = ragged ? ragged_side(d.lanes) : (v == kVarWide ? p.wide_bags : bags_per_tile(var[f]));
         d.tile_begin = static_cast<int32_t>(tiles < INT32_MAX ? tiles : INT32_MAX);
         if (bpt != last_bpt) {  // one division per run of like fields
           last_bpt = bpt;
           field_tiles = (j.batch + bpt - 1) / bpt;
-          if (v == kVarGeneric) field_tiles = (field_tiles + 7) / 8;
+          if (ragged) field_tiles = (field_tiles + 7) / 8;
         }
         tiles += field_tiles;
         d.table = static_cast<const char*>(t.data);
@@ -2215,16 +2213,19 @@ int run_job(const Job& j, hipStream_t stream) {
         d.out_col = t.out_col;
         d.gidx = f;
         const int64_t span = (t.rows - 1) * d.row_bytes + static_cast<int64_t>(t.dim) * tb;
-        const bool pow2 = (d.row_bytes & (d.row_bytes - 1)) == 0;
-        // buffer path: power-of-two rows of >= 8 bytes and (rows + 1) * row_bytes <= 2^32, so the
-        // pad row id 0xffffffff >> log2(row_bytes) addresses past both the rows and the scales
-        const bool fits = d.row_bytes >= 8 && t.rows < (int64_t{1} << 32) / d.row_bytes;
-        const bool ragged_buf = v == kVarGeneric && ragged_buffer_loads(reinterpret_cast<uintptr_t>(t.data), t.rows,
-                                                                        d.row_bytes, t.dim, tb);
-        d.span_bytes = (v == kVarGeneric ? ragged_buf : pow2 && fits) ? static_cast<uint32_t>(span) : 0u;
+        bool buffers;
+        if (ragged) {
+          buffers = ragged_buffer_loads(reinterpret_cast<uintptr_t>(t.data), t.rows, d.row_bytes, t.dim, tb);
+        } else {
+          // power-of-two rows of >= 8 bytes and (rows + 1) * row_bytes <= 2^32, so the pad row id
+          // 0xffffffff >> log2(row_bytes) addresses past both the rows and the scales
+          buffers = (d.row_bytes & (d.row_bytes - 1)) == 0 && d.row_bytes >= 8 &&
+                    t.rows < (int64_t{1} << 32) >> __builtin_ctzll(static_cast<unsigned long long>(d.row_bytes));
+        }
+        d.span_bytes = buffers ? static_cast<uint32_t>(span) : 0u;
         all_buf = all_buf && d.span_bytes != 0;
       }
-      if (v == kVarGeneric) tiles *= 8;
+      if (ragged) tiles *= 8;
       if (tiles > INT32_MAX)
         return set_error(CTI_EBAG_EUNSUPPORTED, "batch of %lld samples needs more than 2^31 tiles", (long long)j.batch);
       p.buffer_ok = all_buf ? 1 : 0;
