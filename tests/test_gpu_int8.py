@@ -143,6 +143,35 @@ def test_quantizer_chunk_edges(pkg, dev, dt, dim, shift):
         assert torch.equal(q, qr)
 
 
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("dim", [5, 50, 64, 128, 129, 256, 500, 1024, 2056])
+def test_quantizer_infinities_and_nans(pkg, dev, dt, dim):
+    """Rows that are not finite: NaNs are left out of the maximum and become 0, as an infinite row's every
+    element does, in the chunk forms (whose fast rounding every such element has to fail) and in the loop
+    over single elements, which the same rows one element further on take from 129 columns on."""
+    print(f"quantize non-finite dt={dt} dim={dim}", flush=True)
+    rng = np.random.default_rng(dim)
+    big = {"f32": 3e38, "bf16": 3e38, "f16": 6e4}[dt]
+    x = rng.standard_normal((70, dim)).astype(np.float32)
+    for r, bad in enumerate([[np.nan], [np.inf], [-np.inf], [np.nan, np.inf], [big], [-big, np.nan]] * 9):
+        for b in bad:
+            x[r, rng.integers(0, dim)] = b
+    x[60], x[61], x[62] = np.nan, np.inf, -np.inf
+    x[63, :-1], x[64, 1:] = np.nan, 0.0
+    for shift in (0, 1):
+        base = torch.zeros(x.size + shift, dtype=TORCH_DT[dt], device=dev)
+        w = base[shift:].view(x.shape)
+        w.copy_(torch.from_numpy(x))
+        v = w.float().cpu().numpy()
+        with np.errstate(invalid="ignore"):
+            s = np.fmax(np.fmax.reduce(np.abs(v), axis=1, initial=0) * np.float32(1 / 127), np.float32(1e-8))
+            q = np.clip(np.rint(v / s[:, None]), -128, 127)
+        q = np.where(np.isnan(q), 0, q).astype(np.int8)
+        got, scale = pkg.quantize_embedding_int8(w)
+        assert np.array_equal(scale.cpu().numpy().view(np.uint32), s.view(np.uint32)), shift
+        assert np.array_equal(got.cpu().numpy(), q), shift
+
+
 # ------------------------------------------------------------------------------------------------
 # pooling
 # ------------------------------------------------------------------------------------------------
