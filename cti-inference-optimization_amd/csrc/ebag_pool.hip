@@ -84,10 +84,16 @@ namespace {
 //   rounds of R length-ranked bags per tile: 2 / 3 / 4 ran 41.7 / 42.5 / 42.1 us.
 constexpr int kRowsInFlight = 4;
 constexpr int kRounds = 2;
-// bags of a streamed tile of rows of 64 lane vectors (kRounds in a launch with a dispatch order, which
-// counts tiles of that many): 28 slots of 512 int8, 4,096 samples, pooled and normalised, 2 / 4 / 8 ran
-// 136 / 131 / 134 us (ranked tiles: 148)
+// bags of a streamed tile of rows of 64 lane vectors, and of one in a launch whose bags are few and long
+// enough that the longest tile sets its time (also in a launch with a dispatch order, which counts tiles of
+// that many). us of 28 slots of 512 int8 pooled at 2 / 4 / 8 bags (ranked tiles): 4,096 samples of mean length
+// 2: 50 / 45 / 46 (52), 8: 102 / 102 / 104 (112); 1,024 samples of 1: 12.1 / 10.4 / 11.0 (12.5), 8: 32.6 /
+// 35.0 / 39.1 (34.7); 128 samples of 8: 13.0 / 14.5 / 18.6 (14.7). bf16, 1,024 samples of 8: 42.9 / 45.1 / 44.6
+// (48.0).
 constexpr int kWideBags = 4;
+constexpr int kWideBagsFew = kRounds;
+// ... at most this many bags (tiles of four then leave wavefront slots of the chip empty), longer than this
+constexpr int64_t kWideFew = 4 * 8192, kWideFewLen = 3;
 
 constexpr int kMainThreads = kWave;  // main kernel: one wavefront per workgroup
 constexpr int kBinThreads = 256;
@@ -2078,7 +2084,7 @@ static_assert(StreamShape<float, 1 << kVarStream, 1>::ok && StreamShape<bf16_t, 
 // walks / id offsets that fit 32 bits.
 bool stream_ids_ok(int64_t nnz, int idx32) {
   constexpr int64_t nb = 8;  // bags per walk, each of which may hold every id (overlapping bags)
-  static_assert(kRounds * (kWave / 16) <= nb && kWideBags <= nb && kFusedBags / fused_waves(kWave) <= nb, "bags per walk");
+  static_assert(kRounds * (kWave / 16) <= nb && kWideBags <= nb && TileShape<float, kWave, 1>::NB == kWideBagsFew && kWideBagsFew <= kWideBags && kFusedBags / fused_waves(kWave) <= nb, "bags per walk");
   return nnz < INT32_MAX / nb && nnz * (idx32 ? 4 : 8) < (int64_t{1} << 32);
 }
 bool stream_variant_allowed(const Job& j) {
@@ -2188,7 +2194,8 @@ int run_job(const Job& j, hipStream_t stream) {
       }
       const size_t nf = fields.size() - c0 < static_cast<size_t>(kMaxFields) ? fields.size() - c0 : kMaxFields;
       p.num_fields = static_cast<int32_t>(nf);
-      p.wide_bags = p.stream_ok && !ordered ? kWideBags : bags_per_tile(kVarWide);
+      const bool wide_few = j.batch <= kWideFew / static_cast<int64_t>(nf) && j.nnz / kWideFewLen > j.batch * j.num_fields;
+      p.wide_bags = p.stream_ok && !ordered && !wide_few ? kWideBags : kWideBagsFew;
       bool all_buf = true;
       int64_t tiles = 0, field_tiles = 0;
       int last_bpt = 0;

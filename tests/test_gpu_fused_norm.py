@@ -171,7 +171,7 @@ def test_encoder_normalized_uses_fused_path(pkg, dev):
                       enc.input_norm.bias.detach(), B, "sum", "bf16"), "bf16")
 
 
-# rows of 64 lane vectors are streamed: tiles of 4 bags (2 with a dispatch order), tables read through
+# rows of 64 lane vectors are streamed: tiles of 4 bags (2 of few long ones or with a dispatch order), tables read through
 # buffers below 4 GiB and with power-of-two rows, else at 64-bit addresses
 @pytest.mark.parametrize("tdt", ["bf16", "f32", "f16", "i8"])
 @pytest.mark.parametrize("B", [1, 4, 5, 67])
