@@ -1895,6 +1895,8 @@ constexpr int64_t kSubThreshold = 24;
 // 48 too: 24 measured 41.7 against 40.7 us there.
 constexpr int64_t kSubThresholdBinned = 48;
 constexpr int64_t kFusedSubThreshold = 48;
+// Rows of 64 lane vectors: mean bag length above which the fused LayerNorm's wavefronts walk.
+constexpr int64_t kFusedWalkLen = 4;
 
 int64_t default_sub_threshold(int variant, bool bins) {
   if (variant == kVarGeneric) return kNoLimit;  // the ragged kernel never splits
@@ -2445,7 +2447,10 @@ int run_fused_norm(const void* values, int32_t index_type, const void* val_offse
   p.num_fields = num_slots;
   p.stream_out = batch_size * p.out_row_stride * tb >= kStreamOutBytes;
   p.sub_threshold = kFusedSubThreshold;
-  p.stream_ok = stream_ids_ok(nnz, p.idx32);
+  // Walk or rounds: the walk keeps more rows in flight, the rounds more wavefronts on a CU. us of 28 slots of 512
+  // bf16, rounds | walk, at mean lengths 2 / 4 / 5 / 8: 4,096 samples 67 | 70, 107 | 107, 118 | 117, 158 | 153; 1,024
+  // samples 23.0 | 24.0, 30.4 | 33.0, 35.4 | 37.2, 49.1 | 47.5; 512 samples 21, 21, 22.8 | 21.7, 31.7 | 28.1.
+  p.stream_ok = stream_ids_ok(nnz, p.idx32) && (int8 || nnz / kFusedWalkLen > batch_size * num_slots);
   p.block_threshold = kNoLimit;
   p.split_threshold = kNoLimit;
   const int64_t rows = max_idx + 1;
