@@ -28,11 +28,12 @@
 //     completes under the current chunk's row loads. Tables under 4 GiB with power-of-two row sizes are read with buffer
 //     loads: a row's offset is one shift-add, and rows past a bag's end use an out-of-range offset
 //     that returns zeros without a memory request (no per-row branch).
-//   * Streamed tiles (256-byte rows of fp32 / bf16 / fp16 tables and 128-byte rows of int8 tables,
-//     without binning and with the default short-bag limit): the same tiles, but the wavefront
-//     walks the tile's rows in order across bag boundaries (with well-formed offsets they are one
-//     contiguous run of `values`), each lane holding 4 bytes (int8: 2 bytes and the row's scale)
-//     of every row, one row per load instruction, 16 rows in flight;
+//   * Streamed tiles (256-byte and 1 KB rows of fp32 / bf16 / fp16 tables, 128- and 512-byte rows of
+//     int8 tables, without binning and with the default short-bag limit): tiles of consecutive bags
+//     again (of 1 KB rows two or four), but the wavefront walks the tile's rows in order across bag
+//     boundaries (with well-formed offsets they are one contiguous run of `values`), each lane
+//     holding 4 bytes (int8: 2 bytes and the row's scale; rows of 64 lane vectors: one vector) of
+//     every row, one row per load instruction, 16 rows in flight (8 of the wide ones);
 //     a bag is stored when its last row has been added, so every bag, whatever its length, is a
 //     sequential fp32 sum in element order. Row ids come one 64-row chunk at a time through
 //     buffer loads over `values` (the next chunk in flight) and are broadcast with readlane.
@@ -137,7 +138,10 @@ struct FieldDesc {
   int32_t out_col;     // first output column
   int32_t gidx;        // field index used for offsets / val_base
   uint32_t span_bytes; // bytes from row 0 to the end of the last row, when below 4 GiB (else 0)
-  int32_t lanes;       // mixed-width launches: log2 of the field's lanes (one vector each); ragged: its chunks
+  union {
+    int32_t lanes_log2;  // mixed-width launches: rows are 1 << lanes_log2 lanes of one vector
+    int32_t chunks;      // ragged launches: chunks of a row
+  };
   int32_t tile_begin;  // mixed-width and ragged launches: the field's first tile (fields in tile order)
 };
 
@@ -1060,7 +1064,7 @@ __global__ void __launch_bounds__(kMainThreads) pool_kernel(const PoolParams p) 
 }
 
 // Main kernel of a mixed-width launch: the fields' rows differ in width but each is one lane
-// vector per lane (LANES = 1 << lanes). Fields own consecutive ranges of tiles; a workgroup
+// vector per lane (LANES = 1 << lanes_log2). Fields own consecutive ranges of tiles; a workgroup
 // finds its tile's field (one compare per lane and a ballot) and runs that width's tile code, so
 // fields of every width share one launch (and one binning pass and one list kernel).
 template <typename TT, typename OT, bool BUF>
@@ -1078,7 +1082,7 @@ __global__ void __launch_bounds__(kMainThreads) pool_mixed_kernel(const PoolPara
   const int first = lane < p.num_fields ? p.f[lane].tile_begin : INT32_MAX;
   const int fi = __popcll(__ballot(first <= tile)) - 1;  // field 0 starts at tile 0
   const int local = tile - p.f[fi].tile_begin;
-  switch (p.f[fi].lanes) {
+  switch (p.f[fi].lanes_log2) {
     case 2: pool_tile<TT, OT, 4, 1, BUF>(p, fi, local, s.l2); break;
     case 3: pool_tile<TT, OT, 8, 1, BUF>(p, fi, local, s.l3); break;
     case 4: pool_tile<TT, OT, 16, 1, BUF>(p, fi, local, s.l4); break;
@@ -1514,15 +1518,15 @@ __device__ __forceinline__ void store_bag_rt(const PoolParams& p, int64_t b, int
   store_out<VEC>(reinterpret_cast<OT*>(p.out) + b * p.out_row_stride + out_col + sl * VEC, r, p.stream_out);
 }
 
-// ... or, in a mixed launch, each field's own (one lane vector per lane, 1 << lanes lanes
-// per row, kMixedLo <= lanes <= kMixedHi), chosen at run time.
+// ... or, in a mixed launch, each field's own (one lane vector per lane, 1 << lanes_log2 lanes
+// per row, kMixedLo <= lanes_log2 <= kMixedHi), chosen at run time.
 template <typename TT, typename OT, int LW>
 struct MixedRows {
   static constexpr int VEC = Elem<TT>::kVecBytes / Elem<TT>::kBytes;
   static constexpr int DMAX = Shape<TT, 1 << kMixedHi, 1>::D;
   __device__ static __forceinline__ void split(const PoolParams& p, int fi, int64_t b, int64_t bs, int64_t be,
                                                int wave, float* s_red, unsigned int* ids) {
-    const int ll = p.f[fi].lanes;
+    const int ll = p.f[fi].lanes_log2;
     const int D = VEC << ll;
     const int sl = lane_id() & ((1 << ll) - 1);
     const bool g0 = lane_id() < (1 << ll);
@@ -1553,7 +1557,7 @@ struct MixedRows {
   }
   __device__ static __forceinline__ void one(const PoolParams& p, int fi, int64_t b, int64_t bs, int64_t be,
                                              unsigned int* ids) {
-    const int ll = p.f[fi].lanes;
+    const int ll = p.f[fi].lanes_log2;
     float pa[VEC];
 #pragma unroll
     for (int i = 0; i < VEC; ++i) pa[i] = 0.f;
@@ -1733,7 +1737,7 @@ __device__ __forceinline__ void ragged_tile(const PoolParams& p, int fi, int loc
   const int64_t max_row = p.f[fi].max_row;
   const int64_t row_bytes = p.f[fi].row_bytes;
   const int dim = p.f[fi].dim;
-  const int chunks = p.f[fi].lanes;
+  const int chunks = p.f[fi].chunks;
   const int n = chunks < kWave ? chunks : kWave;
   const int R = ragged_side(chunks);
   const int lq_max = 31 - __builtin_clz(static_cast<unsigned>(kRaggedIds / R));
@@ -1868,7 +1872,7 @@ __global__ void __launch_bounds__(kMainThreads) pool_ragged_kernel(const PoolPar
   const int fi = __popcll(__ballot(first <= pos)) - 1;  // field 0 starts at position 0
   const int next = fi + 1 < p.num_fields ? p.f[fi + 1].tile_begin : p.num_tiles >> 3;
   const int local = x * (next - p.f[fi].tile_begin) + pos - p.f[fi].tile_begin;
-  if (static_cast<int64_t>(local) * ragged_side(p.f[fi].lanes) >= p.batch) return;  // up to 7 per field
+  if (static_cast<int64_t>(local) * ragged_side(p.f[fi].chunks) >= p.batch) return;  // up to 7 per field
   if constexpr (!Quantized<TT>::value) {
     if (p.f[fi].span_bytes) return ragged_tile<TT, OT, ragged_vec<TT>(), true>(p, fi, local, s);
   }
@@ -2205,8 +2209,9 @@ int run_job(const Job& j, hipStream_t stream) {
         const int f = fields[c0 + i];
         const cti_ebag_table& t = j.tables[f];
         FieldDesc& d = p.f[i];
-        d.lanes = ragged ? ragged_chunks(t.dim, tb == 1 ? 8 : 16 / tb) : (var[f] <= 6 ? var[f] : 0);
-        const int bpt = ragged ? ragged_side(d.lanes) : (v == kVarWide ? p.wide_bags : bags_per_tile(var[f]));
+        if (ragged) d.chunks = ragged_chunks(t.dim, tb == 1 ? 8 : 16 / tb);
+        else d.lanes_log2 = var[f] <= 6 ? var[f] : 0;
+        const int bpt = ragged ? ragged_side(d.chunks) : (v == kVarWide ? p.wide_bags : bags_per_tile(var[f]));
         d.tile_begin = static_cast<int32_t>(tiles < INT32_MAX ? tiles : INT32_MAX);
         if (bpt != last_bpt) {  // one division per run of like fields
           last_bpt = bpt;
@@ -2415,6 +2420,8 @@ int run_fused_norm(const void* values, int32_t index_type, const void* val_offse
   const int tb = dtype_bytes(dtype);
   const int64_t row_bytes = static_cast<int64_t>(emb_dim) * tb;  // of a pooled row
   const int64_t table_row = int8 ? emb_dim : row_bytes;
+  // int8 rows are walked: one 8-byte vector per lane. Narrower rows would need rounds with a scale per row, which
+  // the fused kernel has not; they take two launches.
   if (int8 && (dtype != CTI_EBAG_BF16 || emb_dim != 8 * kWave || !stream_ids_ok(nnz, index_type == CTI_EBAG_I32)))
     return set_error(CTI_EBAG_EUNSUPPORTED, "fused LayerNorm: int8 tables of other than %d columns, rows of another type than "
                      "bf16, or a batch of 2^28 or more ids", 8 * kWave);

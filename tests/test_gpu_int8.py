@@ -339,8 +339,8 @@ def test_int8_plan_and_encoder(pkg, dev):
 
 @pytest.mark.parametrize("D", [1, 3, 8, 24, 100, 136, 4096])
 def test_int8_any_width(pkg, dev, D):
-    """Widths that are not whole lane vectors (or too wide for the vector kernels) take the
-    element-wise kernel; results are still the oracle's bit for bit (one wavefront per bag)."""
+    """Widths that are not whole lane vectors (or too wide for the vector kernels) take the ragged
+    kernel, several bags side by side in a wavefront; results are still the oracle's bit for bit."""
     print(f"int8 width D={D}", flush=True)
     rng = np.random.default_rng(D)
     tables = int8_tables(rng, 3, [77], [D])

@@ -19,7 +19,7 @@ from test_gpu_parity import TORCH_DT, to_dev, to_np
 pytestmark = pytest.mark.gpu
 
 # widths per table type: the mixed range (64 B - 1 KB rows), narrower rows (own launches) and a
-# width that is not a whole number of lane vectors (element-wise kernel)
+# width that is not a whole number of lane vectors (ragged kernel)
 DIMS = {"bf16": (32, 64, 128, 256, 512, 8, 16, 40),
         "f32": (16, 32, 64, 128, 256, 4, 8, 20),
         "f16": (32, 128, 512, 16, 24)}
