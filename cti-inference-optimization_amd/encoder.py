@@ -107,12 +107,14 @@ class RepEncoder(nn.Module):
         """``linear(input_norm(pooled))`` (online_best/infer.py:1029-1085).
 
         By default the pooled block is normalised in place by the LayerNorm kernel and mapped by
-        ``linear`` (torch's GEMM), the faster order at the encoder shape (B = 4096, Linear
-        3584 -> 512) and at the merged 32,768-sample batch. ``fused_linear=True`` takes the
-        statistics pass and the matrix-core kernel that normalises the pooled block's tiles as it
-        loads them (``layer_norm_linear``, K split over the chip when the rows are few), so the
-        normalised block never reaches memory; at the reference's small warm-up batches the two
-        orders are within a few microseconds of each other. It needs a bf16 table and a bf16
+        ``linear`` (torch's GEMM). ``fused_linear=True`` takes the statistics pass and the
+        matrix-core kernel that normalises the pooled block's tiles as it loads them
+        (``layer_norm_linear``, K split over the chip when the rows are few), so the normalised
+        block never reaches memory. Linear 3584 -> 512: within a few microseconds of each other at
+        the reference's small warm-up batches, the default faster at 4,096 rows (62.8 against 69.5
+        us) and up to 16,384, level from 24,576 on (409.7 against 409.0 us at the merged 32,768
+        samples); 3584 -> 256: ``fused_linear`` faster from 8,192 rows on (149 against 130 us
+        there). It needs a bf16 table and a bf16
         ``linear`` with LayerNorm parameters in bf16 or fp32 (the reference's model after
         ``model.to(bfloat16)``, online_best/infer.py:2797).
         """

@@ -352,9 +352,9 @@ int cti_ebag_fused_all_slots_layernorm(const void* values, int32_t index_type, c
 /*
  * cti_ebag_fused_all_slots_layernorm over an int8 table (rows as cti_ebag_fused_all_slots_int8 pools
  * them: acc = fma(q, scale[row], acc) in element order, the sum rounded to bf16). Covered shapes: rows
- * of 512 columns, bf16 output, gamma and beta of F32 or BF16, S <= 64, fewer than 2^28 ids (and 4 GiB
- * of them), 16-byte aligned weight / out / gamma / beta; otherwise CTI_EBAG_EUNSUPPORTED (run
- * cti_ebag_fused_all_slots_int8 and cti_ebag_layernorm instead).
+ * of 512 columns (one 8-byte vector per lane: streamed), bf16 output, gamma and beta of F32 or BF16,
+ * S <= 64, fewer than 2^28 ids (and 4 GiB of them), 16-byte aligned weight / out / gamma / beta;
+ * otherwise CTI_EBAG_EUNSUPPORTED (run cti_ebag_fused_all_slots_int8 and cti_ebag_layernorm instead).
  */
 int cti_ebag_fused_all_slots_layernorm_int8(const void* values, int32_t index_type, const void* val_offsets,
                                             const void* row_offsets, int32_t offset_type, const int8_t* weight_int8,
@@ -439,8 +439,9 @@ int cti_ebag_layernorm(const void* x, void* y, int64_t rows, int64_t cols, int32
  *   workspace  device scratch of workspace_bytes (16-byte aligned), or NULL / 0: when few rows
  *            would leave CUs idle, K is split over several workgroups per output tile, each
  *            writing fp32 partial products here, and a second launch adds the splits in split
- *            order, adds the bias and rounds once; as many splits are used as the workspace holds
- *            (up to cti_ebag_layernorm_linear_workspace_bytes(...); none without a workspace)
+ *            order, adds the bias and rounds once; where that is faster, and at most as many splits
+ *            as the workspace holds (all it can use: cti_ebag_layernorm_linear_workspace_bytes(...);
+ *            none without a workspace)
  * The normalised block is never written to memory. Deterministic: a given shape and workspace
  * size always takes the same splits and accumulation order (other workspace sizes may differ in
  * the last bits, within fp32 accumulation).
@@ -450,7 +451,8 @@ int cti_ebag_layernorm_linear(const void* x, int64_t rows, int32_t cols, const f
                               int32_t out_features, const void* bias, int32_t bias_dtype, void* y,
                               int32_t y_dtype, void* workspace, int64_t workspace_bytes, void* stream);
 
-/* Bytes of workspace cti_ebag_layernorm_linear uses at most for this shape (0: it never splits). */
+/* Bytes of workspace cti_ebag_layernorm_linear uses at most for this shape, whatever the type of gamma
+ * and beta (0: it never splits). */
 int64_t cti_ebag_layernorm_linear_workspace_bytes(int64_t rows, int32_t cols, int32_t out_features);
 
 #ifdef __cplusplus
