@@ -2159,8 +2159,10 @@ int run_job(const Job& j, hipStream_t stream) {
     } else {
       if (!(present & 1u << v) || (mixed && (mixable & 1u << v))) continue;
       for (int f = 0; f < j.num_fields; ++f) if (var[f] == v) fields.push_back(f);
-      if (ragged)  // narrowest rows first (see pool_ragged_kernel)
-        std::stable_sort(fields.begin(), fields.end(), [&](int a, int b) { return j.tables[a].dim < j.tables[b].dim; });
+      if (ragged)  // narrowest rows first (see pool_ragged_kernel), in job order where they are alike
+        std::sort(fields.begin(), fields.end(), [&](int a, int b) {
+          return j.tables[a].dim != j.tables[b].dim ? j.tables[a].dim < j.tables[b].dim : a < b;
+        });
     }
     for (size_t c0 = 0; c0 < fields.size(); c0 += kMaxFields) {
       PoolParams p;
@@ -2204,19 +2206,22 @@ int run_job(const Job& j, hipStream_t stream) {
       p.wide_bags = p.stream_ok && !ordered && !wide_few ? kWideBags : kWideBagsFew;
       bool all_buf = true;
       int64_t tiles = 0, field_tiles = 0;
-      int last_bpt = 0;
+      int last = 0;  // chunks (ragged) or bags per tile of the field before
       for (size_t i = 0; i < nf; ++i) {
         const int f = fields[c0 + i];
         const cti_ebag_table& t = j.tables[f];
         FieldDesc& d = p.f[i];
-        if (ragged) d.chunks = ragged_chunks(t.dim, tb == 1 ? 8 : 16 / tb);
-        else d.lanes_log2 = var[f] <= 6 ? var[f] : 0;
-        const int bpt = ragged ? ragged_side(d.chunks) : (v == kVarWide ? p.wide_bags : bags_per_tile(var[f]));
         d.tile_begin = static_cast<int32_t>(tiles < INT32_MAX ? tiles : INT32_MAX);
-        if (bpt != last_bpt) {  // one division per run of like fields
-          last_bpt = bpt;
-          field_tiles = (j.batch + bpt - 1) / bpt;
-          if (ragged) field_tiles = (field_tiles + 7) / 8;
+        // tiles are divided out once per run of like fields
+        if (ragged) {
+          d.chunks = ragged_chunks(t.dim, tb == 1 ? 8 : 16 / tb);
+          if (d.chunks != last) field_tiles = ((j.batch + ragged_side(d.chunks) - 1) / ragged_side(d.chunks) + 7) / 8;
+          last = d.chunks;
+        } else {
+          d.lanes_log2 = var[f] <= 6 ? var[f] : 0;
+          const int bpt = v == kVarWide ? p.wide_bags : bags_per_tile(var[f]);
+          if (bpt != last) field_tiles = (j.batch + bpt - 1) / bpt;
+          last = bpt;
         }
         tiles += field_tiles;
         d.table = static_cast<const char*>(t.data);
