@@ -1899,8 +1899,10 @@ constexpr int64_t kSubThreshold = 24;
 // 48 too: 24 measured 41.7 against 40.7 us there.
 constexpr int64_t kSubThresholdBinned = 48;
 constexpr int64_t kFusedSubThreshold = 48;
-// Rows of 64 lane vectors: mean bag length above which the fused LayerNorm's wavefronts walk.
-constexpr int64_t kFusedWalkLen = 4;
+// Rows of 64 lane vectors: mean bag length above which the fused LayerNorm's wavefronts walk, and with three to
+// four workgroups a CU.
+constexpr int64_t kFusedWalkLen = 4, kFusedWalkLenTight = 7;
+constexpr int64_t kCus = 256;
 
 int64_t default_sub_threshold(int variant, bool bins) {
   if (variant == kVarGeneric) return kNoLimit;  // the ragged kernel never splits
@@ -2459,10 +2461,6 @@ int run_fused_norm(const void* values, int32_t index_type, const void* val_offse
   p.num_fields = num_slots;
   p.stream_out = batch_size * p.out_row_stride * tb >= kStreamOutBytes;
   p.sub_threshold = kFusedSubThreshold;
-  // Walk or rounds: the walk keeps more rows in flight, the rounds more wavefronts on a CU. us of 28 slots of 512
-  // bf16, rounds | walk, at mean lengths 2 / 4 / 5 / 8: 4,096 samples 67 | 70, 107 | 107, 118 | 117, 158 | 153; 1,024
-  // samples 23.0 | 24.0, 30.4 | 33.0, 35.4 | 37.2, 49.1 | 47.5; 512 samples 21, 21, 22.8 | 21.7, 31.7 | 28.1.
-  p.stream_ok = stream_ids_ok(nnz, p.idx32) && (int8 || nnz / kFusedWalkLen > batch_size * num_slots);
   p.block_threshold = kNoLimit;
   p.split_threshold = kNoLimit;
   const int64_t rows = max_idx + 1;
@@ -2487,6 +2485,14 @@ int run_fused_norm(const void* values, int32_t index_type, const void* val_offse
   fn.eps = eps;
   const size_t row_lds = static_cast<size_t>(row_bytes * num_slots);
   const int spw = fused_samples(num_slots, row_bytes * num_slots);
+  // Walk or rounds: the walk keeps more rows in flight, but a CU holds three of its workgroups (73 VGPRs) and four
+  // of the rounds' (59), so between three and four workgroups a CU it is a second round of them that the walk adds.
+  // us of 28 slots of 512 bf16, rounds | walk, at mean lengths 2 / 4 / 5 / 6 / 8: 4,096 samples 74 | 75, 107 | 107,
+  // 118 | 117, 131 | 129, 158 | 153; 1,024 samples 23.0 | 24.0, 30.4 | 33.0, 35.4 | 37.2, 41.3 | 41.0, 49.1 | 47.5;
+  // 768 samples 21.0 | 21.0, 25.6 | 24.2, 29.4 | 27.1, 34.1 | 29.9, 40.7 | 36.6.
+  const int64_t wgs = (batch_size + spw - 1) / spw;
+  const int64_t walk_len = wgs > 3 * kCus && wgs <= 4 * kCus ? kFusedWalkLenTight : kFusedWalkLen;
+  p.stream_ok = stream_ids_ok(nnz, p.idx32) && (int8 || nnz / walk_len > batch_size * num_slots);
   hipStream_t st = static_cast<hipStream_t>(stream);
   hipError_t e;
   if (int8)
